@@ -125,6 +125,8 @@ __device__ __forceinline__ uint64_t pow7(uint64_t x)
     return p2_mul(x3, x4);
 }
 
+#include "p2_partial.h"
+
 // x^7 on three lanes, each product interleaved across the lanes
 __device__ __forceinline__ void pow7_3(const uint64_t *x, uint64_t *out)
 {
@@ -190,6 +192,7 @@ __device__ __forceinline__ hz sum_halves(const uint64_t *s)
     return a;
 }
 
+// The permutation on one lane alone (the transcript's sponge).
 template <int W>
 __device__ __forceinline__ void p2_permute(uint64_t *s)
 {
@@ -224,6 +227,97 @@ __device__ __forceinline__ void p2_permute(uint64_t *s)
     fold_all<W>(t, s);
 }
 
+// out[i] = s[i]^7, three lanes at a time
+template <int W>
+__device__ __forceinline__ void sbox_all(const uint64_t *s, uint64_t *out)
+{
+    constexpr int G = W / 3 * 3;
+#pragma unroll
+    for (int i = 0; i < G; i += 3) pow7_3(s + i, out + i);
+#pragma unroll
+    for (int i = G; i < W; i++) out[i] = pow7(s[i]);
+}
+
+// Words 0 .. 3 of M_E x, as words: M4 of the block sums 2 x_0 + x_1 + ... (56
+// instructions at width 12 against 148 for the whole layer and its folds).
+template <int W>
+__device__ __forceinline__ void ext_layer_first4(const uint64_t *x, uint64_t *out)
+{
+    hz z[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        z[k].lo = 2ull * (uint32_t)x[k] + (uint32_t)x[4 + k];
+        z[k].hi = 2ull * (uint32_t)(x[k] >> 32) + (uint32_t)(x[4 + k] >> 32);
+#pragma unroll
+        for (int j = 2; j < W / 4; j++) {
+            z[k].lo += (uint32_t)x[4 * j + k];
+            z[k].hi += x[4 * j + k] >> 32;
+        }
+    }
+    hz y[4];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        uint64_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = h ? z[k].hi : z[k].lo;
+        uint64_t t0 = v[0] + v[1], t1 = v[2] + v[3], t2 = (v[1] << 1) + t1, t3 = (v[3] << 1) + t0;
+        uint64_t t4 = (t1 << 2) + t3, t5 = (t0 << 2) + t2;
+        uint64_t o[4] = {t3 + t5, t5, t2 + t4, t4};
+#pragma unroll
+        for (int k = 0; k < 4; k++) (h ? y[k].hi : y[k].lo) = o[k];
+    }
+    hz_fold3(y, out);
+    out[3] = hz_fold(y[3]);
+}
+
+// The permutation with its partial rounds on the matrix cores (p2_partial.h). ops: the
+// lane's operand row in LDS (p2_operand_row). ALL: every word of the result is wanted,
+// otherwise words 0 .. 3 (a digest or the next block's capacity). All 64 lanes of the
+// wave must be active.
+template <int W, bool ALL = false>
+__device__ __forceinline__ void p2_permute_mx(uint64_t *s, const p2_v4i *ops)
+{
+    hz t[W];
+    ext_layer_hz<W>(s, t);
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        uint64_t rc = P2Tab<W>::rc(i);
+        t[i].lo += (uint32_t)rc;
+        t[i].hi += rc >> 32;
+    }
+    fold_all<W>(t, s);
+#pragma unroll 1
+    for (int r = 0; r < (ALL ? 8 : 7); r++) {
+        uint64_t x[W];
+        sbox_all<W>(s, x);
+        ext_layer_hz<W>(x, t);
+        // row r: the constants that follow full round r (none after the last one, and one
+        // before the partial rounds: adding the zeros is less than a branch's copies)
+        const uint64_t *rc = c_p2_next_rc<W>.k[r];
+#pragma unroll
+        for (int i = 0; i < W; i++) {
+            t[i].lo += (uint32_t)rc[i];
+            t[i].hi += rc[i] >> 32;
+        }
+        fold_all<W>(t, s);
+        if (r == 3) {
+#pragma unroll 1
+            for (int g = 0; g < P2_SEGS; g++) p2_segment<W>(s, ops, g);
+        }
+    }
+    if (!ALL) {
+        uint64_t x[W];
+        sbox_all<W>(s, x);
+        ext_layer_first4<W>(x, s);
+    }
+}
+
+// Threads of a block of one-lane permutations. Four waves a SIMD (128 VGPRs) are what the
+// registers allow; the operands in LDS take 19, 30 and 43 KB at widths 8, 12 and 16, so
+// 16 has two blocks of 512 a CU (four blocks of 256 do not fit: 3.9 against 4.1 ms for
+// 2^20 x 128), the others four of 256, which spread short levels over more CUs.
+constexpr __host__ __device__ unsigned p2_threads(unsigned width) { return width == 16 ? 512 : 256; }
+
 // ------------------------------------------------------------ leaves ----
 // Row r of the source: element c at src[r*rs + c*cs]. Digest to out[r*4 .. r*4+3].
 // carry != 0 continues a sponge over later columns: the capacity starts from
@@ -231,30 +325,37 @@ __device__ __forceinline__ void p2_permute(uint64_t *s)
 // columns, which is what the next block's capacity takes), so absorbing a row's
 // columns in groups whose widths are multiples of the rate gives the one-call
 // digest.
+//
+// Bound by VALU issue (2^20 rows x 128 columns at width 12: 8,000 issue slots a wave and
+// permutation, 89 % of the cycles, against 11,300 and 94 % with the partial rounds on the
+// VALU: 5.4 -> 4.35 ms) and by the power that sets the clock (2.0 GHz). Lanes past the
+// last row work on it again, since every lane of a wave holds part of the operands.
 template <int W>
-__global__ __launch_bounds__(P2_THREADS) void k_p2_leaves(const uint64_t *__restrict__ src, uint64_t rs, uint64_t cs,
-                                                          uint64_t ncols, uint64_t nrows, uint64_t *__restrict__ out,
-                                                          uint32_t carry)
+__global__ __launch_bounds__(p2_threads(W), 4) void k_p2_leaves(const uint64_t *__restrict__ src, uint64_t rs,
+                                                                uint64_t cs, uint64_t ncols, uint64_t nrows,
+                                                                uint64_t *__restrict__ out, uint32_t carry)
 {
     constexpr int RATE = W - 4;
-    uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrows) return;
-    uint64_t s[W];
-    const uint64_t *row = src + r * rs;
-#pragma unroll
-    for (int i = RATE; i < W; i++) s[i] = carry ? out[r * 4 + (i - RATE)] : 0;
+    __shared__ p2_v4i ops_s[sizeof(p2c::Operands<W>::b) / 16];
+    const uint64_t r0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (ncols == 0) {
-        if (!carry) {
+        if (r0 < nrows && !carry) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) out[r * 4 + i] = 0;
+            for (int i = 0; i < 4; i++) out[r0 * 4 + i] = 0;
         }
         return;
     }
-    for (uint64_t c0 = 0; c0 < ncols; c0 += RATE) {
-        if (c0 > 0) {
+    p2_operands_load<W>(ops_s);
+    __syncthreads();
+    const p2_v4i *ops = p2_operand_row(ops_s);
+    const uint64_t r = r0 < nrows ? r0 : nrows - 1;
+    uint64_t s[W];
+    const uint64_t *row = src + r * rs;
 #pragma unroll
-            for (int i = 0; i < 4; i++) s[RATE + i] = s[i];
-        }
+    for (int i = 0; i < 4; i++) s[i] = carry ? out[r * 4 + i] : 0;
+    for (uint64_t c0 = 0; c0 < ncols; c0 += RATE) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[RATE + i] = s[i];
         if (c0 + RATE <= ncols) {
 #pragma unroll
             for (int i = 0; i < RATE; i++) s[i] = row[(c0 + i) * cs];
@@ -262,10 +363,12 @@ __global__ __launch_bounds__(P2_THREADS) void k_p2_leaves(const uint64_t *__rest
 #pragma unroll
             for (int i = 0; i < RATE; i++) s[i] = (c0 + i < ncols) ? row[(c0 + i) * cs] : 0;
         }
-        p2_permute<W>(s);
+        p2_permute_mx<W>(s, ops);
     }
+    if (r0 < nrows) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) out[r * 4 + i] = gl_canon(s[i]);
+        for (int i = 0; i < 4; i++) out[r * 4 + i] = gl_canon(s[i]);
+    }
 }
 
 // ------------------------------------------------------------- nodes ----
@@ -273,12 +376,15 @@ __global__ __launch_bounds__(P2_THREADS) void k_p2_leaves(const uint64_t *__rest
 // zero), parents written to out (= in + (pending + pad)*4). The same kernel
 // also writes the zero pad digests after the children.
 template <int W>
-__global__ __launch_bounds__(P2_THREADS) void k_p2_nodes(uint64_t *__restrict__ tree, uint64_t in_off, uint64_t pending,
-                                                         uint64_t pad, uint64_t nnext)
+__global__ __launch_bounds__(p2_threads(W), 4) void k_p2_nodes(uint64_t *__restrict__ tree, uint64_t in_off,
+                                                               uint64_t pending, uint64_t pad, uint64_t nnext)
 {
     constexpr int ARITY = W / 4;
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nnext) return;
+    __shared__ p2_v4i ops_s[sizeof(p2c::Operands<W>::b) / 16];
+    p2_operands_load<W>(ops_s);
+    __syncthreads();
+    const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t i = i0 < nnext ? i0 : nnext - 1;  // all lanes of a wave stay active
     uint64_t s[W];
     const uint64_t *ch = tree + in_off + i * W;
 #pragma unroll
@@ -287,13 +393,15 @@ __global__ __launch_bounds__(P2_THREADS) void k_p2_nodes(uint64_t *__restrict__ 
 #pragma unroll
         for (int k = 0; k < 4; k++) s[a * 4 + k] = real ? ch[a * 4 + k] : 0;
     }
-    if (i == nnext - 1) {
+    if (i0 == nnext - 1) {
         for (uint64_t z = 0; z < pad * 4; z++) tree[in_off + pending * 4 + z] = 0;
     }
-    p2_permute<W>(s);
-    uint64_t *o = tree + in_off + (pending + pad) * 4 + i * 4;
+    p2_permute_mx<W>(s, p2_operand_row(ops_s));
+    if (i0 < nnext) {
+        uint64_t *o = tree + in_off + (pending + pad) * 4 + i * 4;
 #pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = gl_canon(s[k]);
+        for (int k = 0; k < 4; k++) o[k] = gl_canon(s[k]);
+    }
 }
 
 // ------------------------------------------------- cooperative levels ----
@@ -482,15 +590,17 @@ __global__ __launch_bounds__(P2_THREADS) void k_p2_leaves_coop(const uint64_t *_
 // is valid when permute([c0, c1, c2, i, 0, 0, 0, 0])[0] < 2^(64 - n_bits). One
 // lane per nonce of the window [base, base + count); valid nonces go through an
 // atomic minimum, so a window reports its smallest valid nonce.
-__global__ __launch_bounds__(P2_THREADS) void k_p2_grind(uint64_t c0, uint64_t c1, uint64_t c2, uint64_t level,
-                                                         uint64_t base, uint64_t count,
-                                                         unsigned long long *__restrict__ found)
+__global__ __launch_bounds__(p2_threads(8), 4) void k_p2_grind(uint64_t c0, uint64_t c1, uint64_t c2, uint64_t level,
+                                                               uint64_t base, uint64_t count,
+                                                               unsigned long long *__restrict__ found)
 {
-    uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= count) return;
+    __shared__ p2_v4i ops_s[sizeof(p2c::Operands<8>::b) / 16];
+    p2_operands_load<8>(ops_s);
+    __syncthreads();
+    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t s[8] = {c0, c1, c2, base + k, 0, 0, 0, 0};
-    p2_permute<8>(s);
-    if (gl_canon(s[0]) < level) atomicMin(found, (unsigned long long)(base + k));
+    p2_permute_mx<8>(s, p2_operand_row(ops_s));
+    if (k < count && gl_canon(s[0]) < level) atomicMin(found, (unsigned long long)(base + k));
 }
 
 // --------------------------------------------------------- transcript ----
@@ -553,16 +663,20 @@ __global__ void k_transcript(P2TranscriptState *t, uint64_t *io, uint64_t n, int
 
 // Single permutation over `count` states stored consecutively (W words each).
 template <int W>
-__global__ void k_p2_permute_many(uint64_t *st, uint64_t count)
+__global__ __launch_bounds__(p2_threads(W), 4) void k_p2_permute_many(uint64_t *st, uint64_t count)
 {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
+    __shared__ p2_v4i ops_s[sizeof(p2c::Operands<W>::b) / 16];
+    p2_operands_load<W>(ops_s);
+    __syncthreads();
+    const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t s[W];
 #pragma unroll
-    for (int k = 0; k < W; k++) s[k] = st[i * W + k];
-    p2_permute<W>(s);
+    for (int k = 0; k < W; k++) s[k] = i0 < count ? st[i0 * W + k] : 0;
+    p2_permute_mx<W, true>(s, p2_operand_row(ops_s));
+    if (i0 < count) {
 #pragma unroll
-    for (int k = 0; k < W; k++) st[i * W + k] = gl_canon(s[k]);
+        for (int k = 0; k < W; k++) st[i0 * W + k] = gl_canon(s[k]);
+    }
 }
 
 // ---------------------------------------------------- product peak ----
@@ -652,8 +766,8 @@ extern "C" int p2_launch_grind(const uint64_t *ch, uint64_t level, uint64_t base
                                uint64_t *found, hipStream_t st)
 {
     if (count == 0) return 0;
-    dim3 g((unsigned)((count + P2_THREADS - 1) / P2_THREADS));
-    hipLaunchKernelGGL(k_p2_grind, g, dim3(P2_THREADS), 0, st, ch[0], ch[1], ch[2], level, base, count,
+    dim3 g((unsigned)((count + p2_threads(8) - 1) / p2_threads(8)));
+    hipLaunchKernelGGL(k_p2_grind, g, dim3(p2_threads(8)), 0, st, ch[0], ch[1], ch[2], level, base, count,
                        (unsigned long long *)found);
     return (int)hipGetLastError();
 }
@@ -696,11 +810,12 @@ extern "C" int p2_launch_leaves_carry(uint32_t width, const uint64_t *src, uint6
         }
         return (int)hipGetLastError();
     }
-    dim3 g((unsigned)((nrows + P2_THREADS - 1) / P2_THREADS));
+    const unsigned nt = p2_threads(width);
+    dim3 g((unsigned)((nrows + nt - 1) / nt));
     switch (width) {
-    case 8: hipLaunchKernelGGL(k_p2_leaves<8>, g, dim3(P2_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
-    case 12: hipLaunchKernelGGL(k_p2_leaves<12>, g, dim3(P2_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
-    case 16: hipLaunchKernelGGL(k_p2_leaves<16>, g, dim3(P2_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
+    case 8: hipLaunchKernelGGL(k_p2_leaves<8>, g, dim3(nt), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
+    case 12: hipLaunchKernelGGL(k_p2_leaves<12>, g, dim3(nt), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
+    case 16: hipLaunchKernelGGL(k_p2_leaves<16>, g, dim3(nt), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
     default: return -1;
     }
     return (int)hipGetLastError();
@@ -722,11 +837,12 @@ extern "C" int p2_launch_tree_levels(uint32_t width, uint64_t *tree, uint64_t nl
             default: return -1;
             }
         } else {
-            dim3 g((unsigned)((next + P2_THREADS - 1) / P2_THREADS));
+            const unsigned nt = p2_threads(width);
+            dim3 g((unsigned)((next + nt - 1) / nt));
             switch (width) {
-            case 8: hipLaunchKernelGGL(k_p2_nodes<8>, g, dim3(P2_THREADS), 0, st, tree, off, pending, pad, next); break;
-            case 12: hipLaunchKernelGGL(k_p2_nodes<12>, g, dim3(P2_THREADS), 0, st, tree, off, pending, pad, next); break;
-            case 16: hipLaunchKernelGGL(k_p2_nodes<16>, g, dim3(P2_THREADS), 0, st, tree, off, pending, pad, next); break;
+            case 8: hipLaunchKernelGGL(k_p2_nodes<8>, g, dim3(nt), 0, st, tree, off, pending, pad, next); break;
+            case 12: hipLaunchKernelGGL(k_p2_nodes<12>, g, dim3(nt), 0, st, tree, off, pending, pad, next); break;
+            case 16: hipLaunchKernelGGL(k_p2_nodes<16>, g, dim3(nt), 0, st, tree, off, pending, pad, next); break;
             default: return -1;
             }
         }
@@ -746,11 +862,12 @@ extern "C" int p2_launch_mul_peak(const uint64_t *in, uint64_t *out, uint64_t la
 extern "C" int p2_launch_permute(uint32_t width, uint64_t *states, uint64_t count, hipStream_t st)
 {
     if (count == 0) return 0;
-    dim3 g((unsigned)((count + 127) / 128));
+    const unsigned nt = p2_threads(width);
+    dim3 g((unsigned)((count + nt - 1) / nt));
     switch (width) {
-    case 8: hipLaunchKernelGGL(k_p2_permute_many<8>, g, dim3(128), 0, st, states, count); break;
-    case 12: hipLaunchKernelGGL(k_p2_permute_many<12>, g, dim3(128), 0, st, states, count); break;
-    case 16: hipLaunchKernelGGL(k_p2_permute_many<16>, g, dim3(128), 0, st, states, count); break;
+    case 8: hipLaunchKernelGGL(k_p2_permute_many<8>, g, dim3(nt), 0, st, states, count); break;
+    case 12: hipLaunchKernelGGL(k_p2_permute_many<12>, g, dim3(nt), 0, st, states, count); break;
+    case 16: hipLaunchKernelGGL(k_p2_permute_many<16>, g, dim3(nt), 0, st, states, count); break;
     default: return -1;
     }
     return (int)hipGetLastError();
