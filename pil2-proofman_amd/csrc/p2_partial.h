@@ -14,8 +14,10 @@
 // of the column in each. With A block diagonal over the two lane halves every lane
 // multiplies its own two words: a lane keeps its own permutation, one instruction
 // gives four word products for each of the 64 lanes, and the matrix cores run beside
-// the VALU work of the other waves. (A holds zeros in half of its lanes; spreading a
-// permutation over two lanes would use them, but the S-boxes need it in one.)
+// the VALU work of the other waves. A holds zeros in half of its lanes then; the state
+// after the segment, which no S-box waits for, is computed with words exchanged between
+// lanes l and l + 32 and whole operands (111 -> 81 products a segment at width 12, leaves
+// of 2^20 x 128 rows 4.37 -> 4.10 ms).
 //
 // Bytes are signed in the instruction: words enter as w ^ 0x8080808080808080, i.e.
 // byte - 128, and 128 * (sum of the coefficients) * 0x0101010101010101 goes into the
@@ -63,45 +65,69 @@ template <int W> struct Forms {
 template <int W> inline constexpr Forms<W> forms{};
 
 // The A operands in the order they are used. In-words go in pairs (s_1, s_2), ...,
-// (s_{W-1}, y_0), (y_1, y_2), ..., out-words in pairs too. The pair (u_{2p+1}, u_{2p+2})
-// takes every in-pair up to (y_{2p-1}, y_{2p}) and then (y_{2p+1}, -) for its second
-// word; the state pairs take all of them. All in-pairs of the next out-pair but its last
-// come before that (y_{2p+1}, -). An operand is 16 rows (out-word, digit) of 16 bytes
-// (in-word, byte) and a 17th row of zeros, which the lanes off the diagonal read.
+// (s_{W-1}, y_0), (y_1, y_2), ..., and the u in pairs too: (u_{2p+1}, u_{2p+2}) takes
+// every in-pair up to (y_{2p-1}, y_{2p}) and then (y_{2p+1}, -) for its second word. All
+// in-pairs of the next pair but its last come before that (y_{2p+1}, -). These operands
+// are 16 rows (out-word, digit) of 16 bytes (in-word, byte) and a 17th row of zeros,
+// which the lanes off the diagonal read.
+//
+// The state after the segment takes no part in that chain, so its products use the
+// whole operand: lanes l and l + 32 exchange words (v_permlane32_swap), after which one
+// B operand holds four words of the lower lane's permutation and another four of the
+// upper one's, and one D operand four words of the result, two in each lane. That takes
+// half the products: four out-words of 2 in-pairs are 2 x 2 instead of 2 x 4. In-pairs
+// 2t and 2t + 1 give operand t (an odd last pair is paired with nothing), out-words 4m,
+// 4m + 1 are in lane l, 4m + 2 and 4m + 3 in lane l + 32; 32 rows of 32 bytes.
 template <int W> struct Operands {
     static constexpr int NS = W / 2, NY = (P2_SEG - 1) / 2;  // in-pairs: NS, then NY
-    static constexpr int NU = (P2_SEG - 1) / 2;              // pairs of u, then W / 2 of the state
-    static constexpr int COUNT = NU * NS + NU * (NU - 1) / 2 + NU + (W / 2) * (NS + NY);
+    static constexpr int NU = (P2_SEG - 1) / 2;              // pairs of u
+    static constexpr int COUNT = NS + NU * NS + NU * (NU - 1) / 2 + 2 * NU - NS - NY;  // operands of the u
     static constexpr int STRIDE = 17 * 16;
+    static constexpr int NK = (NS + NY + 1) / 2, NM = W / 4;  // state operands: NM rows of NK
+    static constexpr int STATE = COUNT * STRIDE;              // where they start
     static_assert(Forms<W>::NIN * 8 * 128 * 128 < 1 << 22, "digit sums (p2_digits)");
-    alignas(16) int8_t b[COUNT * STRIDE];
+    alignas(16) int8_t b[STATE + NM * NK * 1024];
+    // the digits of coefficient c times 2^(8a), a < 8: row t, byte a at b[at + t * 16 + a]
+    constexpr void digits(int at, uint64_t c)
+    {
+        uint64_t v = c;
+        for (int a = 0; a < 8; a++, v = mul(v, 256)) {
+            // v or v - p in the range of eight digits -128 .. 127; digit = byte or byte - 256
+            uint64_t x = v > 0x7F7F7F7F7F7F7F7FULL ? v - GL_P : v;
+            for (int t = 0; t < 8; t++) {
+                int64_t d = (int64_t)(int8_t)(x & 255);
+                b[at + t * 16 + a] = (int8_t)d;
+                x = (uint64_t)((int64_t)(x - (uint64_t)d) >> 8);
+            }
+        }
+    }
     constexpr void put(int n, int out0, int in0, bool half)
     {
         for (int o = 0; o < 2; o++)
-            for (int i = 0; i < (half ? 1 : 2); i++) {
-                uint64_t v = half && o == 0 ? 0 : forms<W>.c[out0 + o][in0 + i];
-                for (int a = 0; a < 8; a++, v = mul(v, 256)) {
-                    // v or v - p in the range of eight digits -128 .. 127; digit = byte or byte - 256
-                    uint64_t x = v > 0x7F7F7F7F7F7F7F7FULL ? v - GL_P : v;
-                    for (int t = 0; t < 8; t++) {
-                        int64_t d = (int64_t)(int8_t)(x & 255);
-                        b[n * STRIDE + (o * 8 + t) * 16 + i * 8 + a] = (int8_t)d;
-                        x = (uint64_t)((int64_t)(x - (uint64_t)d) >> 8);
-                    }
-                }
-            }
+            for (int i = 0; i < (half ? 1 : 2); i++)
+                digits(n * STRIDE + o * 8 * 16 + i * 8, half && o == 0 ? 0 : forms<W>.c[out0 + o][in0 + i]);
     }
     constexpr Operands() : b{}
     {
         int n = 0;
         for (int t = 0; t < NS; t++) put(n++, 0, 2 * t, false);
         for (int p = 0; p < NU; p++) {
-            for (int t = 0; t < NS + p; t++) put(n++, 2 * p + 2, 2 * t, false);
+            for (int t = 0; t < NS + p && p + 1 < NU; t++) put(n++, 2 * p + 2, 2 * t, false);
             put(n++, 2 * p, 2 * (NS + p), true);
-            put(n++, 2 * p + 2, 2 * (NS + p), false);
+            if (p + 1 < NU) put(n++, 2 * p + 2, 2 * (NS + p), false);
         }
-        for (int p = NU + 1; p < NU + W / 2; p++)
-            for (int t = 0; t < NS + NY; t++) put(n++, 2 * p, 2 * t, false);
+        // 16-byte pieces: k-half kh of the 16 rows of row half oh at ((kh * 2 + oh) * 16 + row) * 16
+        for (int m = 0; m < NM; m++)
+            for (int k = 0; k < NK; k++)
+                for (int oh = 0; oh < 2; oh++)
+                    for (int o = 0; o < 2; o++)
+                        for (int kh = 0; kh < 2; kh++)
+                            for (int i = 0; i < 2; i++) {
+                                int in = 4 * k + 2 * kh + i;
+                                if (in < Forms<W>::NIN)
+                                    digits(STATE + (m * NK + k) * 1024 + ((kh * 2 + oh) * 16 + o * 8) * 16 + i * 8,
+                                           forms<W>.c[P2_SEG - 1 + 4 * m + 2 * oh + o][in]);
+                            }
     }
 };
 
@@ -160,35 +186,41 @@ __device__ __forceinline__ void p2_operands_load(p2_v4i *s)
     for (uint32_t i = threadIdx.x; i < sizeof(p2c::Operands<W>::b) / 16; i += blockDim.x) s[i] = g[i];
 }
 
-// The lane's first A row in LDS: row l % 32 of the operand for k-half l / 32; its data
-// row is 4 (row / 8) + row % 4 if the row belongs to that half, else the zero row.
-__device__ __forceinline__ const p2_v4i *p2_operand_row(const p2_v4i *s)
+// Where the lane's row l % 32 of the A operands is in LDS, for k-half l / 32: D row
+// 8q + 4h + j is row 4q + j of lane half h. u: the 16 rows of a diagonal operand, for
+// lanes whose row belongs to the other half the zero row; w: of a state operand.
+struct p2_rows {
+    const p2_v4i *u, *w;
+};
+template <int W>
+__device__ __forceinline__ p2_rows p2_operand_rows(const p2_v4i *s)
 {
-    uint32_t l = __lane_id(), row = l & 31;
-    return s + (((row >> 2) & 1) == (l >> 5) ? 4 * (row >> 3) + (row & 3) : 16);
+    uint32_t l = __lane_id(), row = l & 31, kh = l >> 5, oh = (row >> 2) & 1, i = 4 * (row >> 3) + (row & 3);
+    return {s + (oh == kh ? i : 16), s + p2c::Operands<W>::STATE / 16 + (kh * 2 + oh) * 16 + i};
 }
 
 // The result whose eight digit sums (absolute values < 2^22) start at acc[at]: lo + 2^32 hi
-// plus the addends
-__device__ __forceinline__ hz p2_digits(const p2_v16i &acc, int at, const uint64_t *k, uint32_t c16)
-{
-    uint32_t a[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) a[i] = (uint32_t)acc[at + i];
-    uint32_t e0 = (a[1] << 8) + a[0], e1 = (a[3] << 8) + a[2];
-    uint32_t e2 = (a[5] << 8) + a[4], e3 = (a[7] << 8) + a[6];
-    uint64_t l, h, d0, d1;
-    asm("v_mad_i64_i32 %0, %2, %4, %6, %7\n\t"
-        "v_mad_i64_i32 %1, %3, %5, %6, %8"
-        : "=&v"(l), "=&v"(h), "=&s"(d0), "=&s"(d1)
-        : "v"(e1), "v"(e3), "v"(c16), "s"(k[0]), "s"(k[1]));
-    hz r;
-    asm("v_mad_i64_i32 %0, %2, %4, 1, %6\n\t"
-        "v_mad_i64_i32 %1, %3, %5, 1, %7"
-        : "=&v"(r.lo), "=&v"(r.hi), "=&s"(d0), "=&s"(d1)
-        : "v"(e0), "v"(e2), "v"(l), "v"(h));
-    return r;
-}
+// plus the addends k, the same for the wave or (p2_digits_v) each lane's own
+#define P2_DIGITS(NAME, KC)                                                                           \
+    __device__ __forceinline__ hz NAME(const p2_v16i &acc, int at, const uint64_t *k, uint32_t c16)   \
+    {                                                                                                 \
+        uint32_t e[4];                                                                                \
+        _Pragma("unroll") for (int i = 0; i < 4; i++) e[i] =                                          \
+            ((uint32_t)acc[at + 2 * i + 1] << 8) + (uint32_t)acc[at + 2 * i];                         \
+        uint64_t l, h, d0, d1;                                                                        \
+        asm("v_mad_i64_i32 %0, %2, %4, %6, %7\n\t"                                                    \
+            "v_mad_i64_i32 %1, %3, %5, %6, %8"                                                        \
+            : "=&v"(l), "=&v"(h), "=&s"(d0), "=&s"(d1)                                                \
+            : "v"(e[1]), "v"(e[3]), "v"(c16), KC(k[0]), KC(k[1]));                                    \
+        hz r;                                                                                         \
+        asm("v_mad_i64_i32 %0, %2, %4, 1, %6\n\t"                                                     \
+            "v_mad_i64_i32 %1, %3, %5, 1, %7"                                                         \
+            : "=&v"(r.lo), "=&v"(r.hi), "=&s"(d0), "=&s"(d1)                                          \
+            : "v"(e[0]), "v"(e[2]), "v"(l), "v"(h));                                                  \
+        return r;                                                                                     \
+    }
+P2_DIGITS(p2_digits, "s")
+P2_DIGITS(p2_digits_v, "v")
 
 // Bytes of a word as the signed bytes of half an operand
 __device__ __forceinline__ void p2_put_word(p2_v4i &v, int half, uint64_t w)
@@ -197,43 +229,64 @@ __device__ __forceinline__ void p2_put_word(p2_v4i &v, int half, uint64_t w)
     v[2 * half + 1] = (int)((uint32_t)(w >> 32) ^ 0x80808080u);
 }
 
-// The A operands on their way from LDS, P2_AHEAD of them (1 to 5 measure the same within
-// 2 %; more than 2 pushes width 16 over 128 VGPRs).
+// The A operands on their way from LDS, P2_AHEAD of them (1 and 2 measure the same within
+// 2 %; more pushes width 16 further over 128 VGPRs). First those of the u, then the state's.
 #define P2_AHEAD 2
 template <int W> struct p2_stream {
-    const p2_v4i *ops;
+    using Op = p2c::Operands<W>;
+    p2_rows ops;
     p2_v4i a[P2_AHEAD];
     int n;
-    __device__ __forceinline__ void start(const p2_v4i *o)
+    __device__ __forceinline__ void fetch(int i)
+    {
+        if (i < Op::COUNT)
+            a[i % P2_AHEAD] = ops.u[i * 17];
+        else if (i < Op::COUNT + Op::NM * Op::NK)
+            a[i % P2_AHEAD] = ops.w[(i - Op::COUNT) * 64];
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ void start(const p2_rows &o)
     {
         ops = o;
         n = 0;
 #pragma unroll
-        for (int i = 0; i < P2_AHEAD; i++) a[i] = ops[i * 17];
-        asm volatile("" ::: "memory");
+        for (int i = 0; i < P2_AHEAD; i++) fetch(i);
     }
-    // acc += operand n * in; operand n + P2_AHEAD is read
+    // acc += operand n * in
     __device__ __forceinline__ void mac(p2_v16i &acc, const p2_v4i &in)
     {
         acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[n % P2_AHEAD], in, acc, 0, 0, 0);
-        if (n + P2_AHEAD < p2c::Operands<W>::COUNT) a[n % P2_AHEAD] = ops[(n + P2_AHEAD) * 17];
-        asm volatile("" ::: "memory");
+        fetch(n + P2_AHEAD);
         n++;
     }
+    // acc0 += operand n * in0, acc1 += operand n * in1
+    __device__ __forceinline__ void mac2(p2_v16i &acc0, const p2_v4i &in0, p2_v16i &acc1, const p2_v4i &in1)
+    {
+        acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[n % P2_AHEAD], in0, acc0, 0, 0, 0);
+        mac(acc1, in1);
+    }
 };
+
+// x of lanes 32 .. 63 and y of lanes 0 .. 31 change places
+__device__ __forceinline__ void p2_swap32(int &x, int &y)
+{
+    auto r = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    x = (int)r[0];
+    y = (int)r[1];
+}
 
 // One segment on the state s, where s[0] already holds its round constant; s[0] (and
 // after the last segment every word) comes out with the next one. All 64 lanes of the
 // wave must be active: the A operands are spread over them. While an S-box runs, the
-// products of the next out-pair that do not wait for it are under way.
+// products of the next pair of u that do not wait for it are under way.
 template <int W>
-__device__ __forceinline__ void p2_segment(uint64_t *s, const p2_v4i *ops, int g)
+__device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int g)
 {
     using Op = p2c::Operands<W>;
     constexpr int NS = Op::NS, NY = Op::NY, NU = Op::NU;
     const uint64_t(*k)[2] = c_p2_addends<W>.k[g];
     const uint32_t c16 = 65536;
-    p2_v4i in[NS + NY];
+    p2_v4i in[2 * Op::NK];
     p2_stream<W> st;
     st.start(ops);
 #pragma unroll
@@ -248,7 +301,7 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_v4i *ops, int g
         hz u = p2_digits(acc, 0, k[2 * p], c16);
         nxt = (p2_v16i){};
 #pragma unroll
-        for (int t = 0; t < NS + p; t++) st.mac(nxt, in[t]);
+        for (int t = 0; t < NS + p && p + 1 < NU; t++) st.mac(nxt, in[t]);
         uint64_t y = pow7(hz_fold(u));
         p2_put_word(in[NS + p], 0, y);
         p2_put_word(in[NS + p], 1, y);  // any value: its coefficients in the next operand are zero
@@ -258,23 +311,45 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_v4i *ops, int g
         // reserved until its results have been read
         asm volatile("" : "+v"(u.lo) : "v"(acc));
         p2_put_word(in[NS + p], 1, pow7(hz_fold(u)));
-        st.mac(nxt, in[NS + p]);
+        if (p + 1 < NU) st.mac(nxt, in[NS + p]);
         acc = nxt;
     }
+    if ((NS + NY) % 2) in[NS + NY] = in[NS + NY - 1];  // any value: its coefficients are zero
 #pragma unroll
-    for (int p = 0; p < W / 2; p++) {
-        if (p + 1 < W / 2) {
-            nxt = (p2_v16i){};
+    for (int t = 0; t < Op::NK; t++) {
 #pragma unroll
-            for (int t = 0; t < NS + NY; t++) st.mac(nxt, in[t]);
+        for (int i = 0; i < 4; i++) {
+            int x = in[2 * t][i], y = in[2 * t + 1][i];
+            p2_swap32(x, y);
+            in[2 * t][i] = x;
+            in[2 * t + 1][i] = y;
         }
-        s[2 * p] = hz_fold(p2_digits(acc, 0, k[P2_SEG - 1 + 2 * p], c16));
-        s[2 * p + 1] = hz_fold(p2_digits(acc, 8, k[P2_SEG + 2 * p], c16));
-        acc = nxt;
+    }
+    // the state words' addends, those of lane half h at k[.. + 2h]
+    const uint64_t(*kh)[2] = k + P2_SEG - 1 + 2 * (__lane_id() >> 5);
+#pragma unroll
+    for (int m = 0; m < Op::NM; m++) {
+        acc = nxt = (p2_v16i){};
+#pragma unroll
+        for (int t = 0; t < Op::NK; t++) st.mac2(acc, in[2 * t], nxt, in[2 * t + 1]);
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            uint64_t x = hz_fold(p2_digits_v(acc, 8 * o, kh[4 * m + o], c16));
+            uint64_t y = hz_fold(p2_digits_v(nxt, 8 * o, kh[4 * m + o], c16));
+            asm volatile("s_nop 1" : "+v"(x), "+v"(y));  // the exchange reads what inline assembly wrote
+            int x0 = (int)(uint32_t)x, x1 = (int)(x >> 32), y0 = (int)(uint32_t)y, y1 = (int)(y >> 32);
+            p2_swap32(x0, y0);
+            p2_swap32(x1, y1);
+            s[4 * m + o] = gl_pack((uint32_t)x0, (uint32_t)x1);
+            s[4 * m + 2 + o] = gl_pack((uint32_t)y0, (uint32_t)y1);
+        }
     }
 }
 #else  // host pass: declarations only (the kernels are compiled for the device)
 template <int W> __device__ void p2_operands_load(p2_v4i *s);
-__device__ const p2_v4i *p2_operand_row(const p2_v4i *s);
-template <int W> __device__ void p2_segment(uint64_t *s, const p2_v4i *ops, int g);
+struct p2_rows {
+    const p2_v4i *u, *w;
+};
+template <int W> __device__ p2_rows p2_operand_rows(const p2_v4i *s);
+template <int W> __device__ void p2_segment(uint64_t *s, const p2_rows &ops, int g);
 #endif

@@ -271,11 +271,11 @@ __device__ __forceinline__ void ext_layer_first4(const uint64_t *x, uint64_t *ou
 }
 
 // The permutation with its partial rounds on the matrix cores (p2_partial.h). ops: the
-// lane's operand row in LDS (p2_operand_row). ALL: every word of the result is wanted,
+// lane's operand rows in LDS (p2_operand_rows). ALL: every word of the result is wanted,
 // otherwise words 0 .. 3 (a digest or the next block's capacity). All 64 lanes of the
 // wave must be active.
 template <int W, bool ALL = false>
-__device__ __forceinline__ void p2_permute_mx(uint64_t *s, const p2_v4i *ops)
+__device__ __forceinline__ void p2_permute_mx(uint64_t *s, const p2_rows &ops)
 {
     hz t[W];
     ext_layer_hz<W>(s, t);
@@ -312,11 +312,13 @@ __device__ __forceinline__ void p2_permute_mx(uint64_t *s, const p2_v4i *ops)
     }
 }
 
-// Threads of a block of one-lane permutations. Four waves a SIMD (128 VGPRs) are what the
-// registers allow; the operands in LDS take 19, 30 and 43 KB at widths 8, 12 and 16, so
-// 16 has two blocks of 512 a CU (four blocks of 256 do not fit: 3.9 against 4.1 ms for
-// 2^20 x 128), the others four of 256, which spread short levels over more CUs.
-constexpr __host__ __device__ unsigned p2_threads(unsigned width) { return width == 16 ? 512 : 256; }
+// Threads of a block of one-lane permutations, n of them. Four waves a SIMD (128 VGPRs)
+// are what the registers allow; the operands in LDS take 19, 30 and 43 KB at widths 8, 12
+// and 16, so width 16 reaches them with two blocks of 512 a CU only (3.72 against 3.84 ms
+// for 2^20 x 128). Blocks of 256 put one wave on each SIMD of up to 256 CUs, which is
+// faster up to 2^16 permutations (20,000 rows x 13: 0.086 against 0.102 ms).
+constexpr __host__ __device__ unsigned p2_max_threads(unsigned width) { return width == 16 ? 512 : 256; }
+static inline unsigned p2_threads(unsigned width, uint64_t n) { return n > 65536 ? p2_max_threads(width) : 256; }
 
 // ------------------------------------------------------------ leaves ----
 // Row r of the source: element c at src[r*rs + c*cs]. Digest to out[r*4 .. r*4+3].
@@ -326,12 +328,12 @@ constexpr __host__ __device__ unsigned p2_threads(unsigned width) { return width
 // columns in groups whose widths are multiples of the rate gives the one-call
 // digest.
 //
-// Bound by VALU issue (2^20 rows x 128 columns at width 12: 8,000 issue slots a wave and
+// Bound by VALU issue (2^20 rows x 128 columns at width 12: 7,900 issue slots a wave and
 // permutation, 89 % of the cycles, against 11,300 and 94 % with the partial rounds on the
-// VALU: 5.4 -> 4.35 ms) and by the power that sets the clock (2.0 GHz). Lanes past the
+// VALU: 5.4 -> 4.10 ms) and by the power that sets the clock (2.0 GHz). Lanes past the
 // last row work on it again, since every lane of a wave holds part of the operands.
 template <int W>
-__global__ __launch_bounds__(p2_threads(W), 4) void k_p2_leaves(const uint64_t *__restrict__ src, uint64_t rs,
+__global__ __launch_bounds__(p2_max_threads(W), 4) void k_p2_leaves(const uint64_t *__restrict__ src, uint64_t rs,
                                                                 uint64_t cs, uint64_t ncols, uint64_t nrows,
                                                                 uint64_t *__restrict__ out, uint32_t carry)
 {
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(p2_threads(W), 4) void k_p2_leaves(const uint64_t *
     }
     p2_operands_load<W>(ops_s);
     __syncthreads();
-    const p2_v4i *ops = p2_operand_row(ops_s);
+    const p2_rows ops = p2_operand_rows<W>(ops_s);
     const uint64_t r = r0 < nrows ? r0 : nrows - 1;
     uint64_t s[W];
     const uint64_t *row = src + r * rs;
@@ -376,7 +378,7 @@ __global__ __launch_bounds__(p2_threads(W), 4) void k_p2_leaves(const uint64_t *
 // zero), parents written to out (= in + (pending + pad)*4). The same kernel
 // also writes the zero pad digests after the children.
 template <int W>
-__global__ __launch_bounds__(p2_threads(W), 4) void k_p2_nodes(uint64_t *__restrict__ tree, uint64_t in_off,
+__global__ __launch_bounds__(p2_max_threads(W), 4) void k_p2_nodes(uint64_t *__restrict__ tree, uint64_t in_off,
                                                                uint64_t pending, uint64_t pad, uint64_t nnext)
 {
     constexpr int ARITY = W / 4;
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(p2_threads(W), 4) void k_p2_nodes(uint64_t *__restr
     if (i0 == nnext - 1) {
         for (uint64_t z = 0; z < pad * 4; z++) tree[in_off + pending * 4 + z] = 0;
     }
-    p2_permute_mx<W>(s, p2_operand_row(ops_s));
+    p2_permute_mx<W>(s, p2_operand_rows<W>(ops_s));
     if (i0 < nnext) {
         uint64_t *o = tree + in_off + (pending + pad) * 4 + i * 4;
 #pragma unroll
@@ -590,7 +592,7 @@ __global__ __launch_bounds__(P2_THREADS) void k_p2_leaves_coop(const uint64_t *_
 // is valid when permute([c0, c1, c2, i, 0, 0, 0, 0])[0] < 2^(64 - n_bits). One
 // lane per nonce of the window [base, base + count); valid nonces go through an
 // atomic minimum, so a window reports its smallest valid nonce.
-__global__ __launch_bounds__(p2_threads(8), 4) void k_p2_grind(uint64_t c0, uint64_t c1, uint64_t c2, uint64_t level,
+__global__ __launch_bounds__(p2_max_threads(8), 4) void k_p2_grind(uint64_t c0, uint64_t c1, uint64_t c2, uint64_t level,
                                                                uint64_t base, uint64_t count,
                                                                unsigned long long *__restrict__ found)
 {
@@ -599,7 +601,7 @@ __global__ __launch_bounds__(p2_threads(8), 4) void k_p2_grind(uint64_t c0, uint
     __syncthreads();
     const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t s[8] = {c0, c1, c2, base + k, 0, 0, 0, 0};
-    p2_permute_mx<8>(s, p2_operand_row(ops_s));
+    p2_permute_mx<8>(s, p2_operand_rows<8>(ops_s));
     if (k < count && gl_canon(s[0]) < level) atomicMin(found, (unsigned long long)(base + k));
 }
 
@@ -663,7 +665,7 @@ __global__ void k_transcript(P2TranscriptState *t, uint64_t *io, uint64_t n, int
 
 // Single permutation over `count` states stored consecutively (W words each).
 template <int W>
-__global__ __launch_bounds__(p2_threads(W), 4) void k_p2_permute_many(uint64_t *st, uint64_t count)
+__global__ __launch_bounds__(p2_max_threads(W), 4) void k_p2_permute_many(uint64_t *st, uint64_t count)
 {
     __shared__ p2_v4i ops_s[sizeof(p2c::Operands<W>::b) / 16];
     p2_operands_load<W>(ops_s);
@@ -672,7 +674,7 @@ __global__ __launch_bounds__(p2_threads(W), 4) void k_p2_permute_many(uint64_t *
     uint64_t s[W];
 #pragma unroll
     for (int k = 0; k < W; k++) s[k] = i0 < count ? st[i0 * W + k] : 0;
-    p2_permute_mx<W, true>(s, p2_operand_row(ops_s));
+    p2_permute_mx<W, true>(s, p2_operand_rows<W>(ops_s));
     if (i0 < count) {
 #pragma unroll
         for (int k = 0; k < W; k++) st[i0 * W + k] = gl_canon(s[k]);
@@ -766,8 +768,9 @@ extern "C" int p2_launch_grind(const uint64_t *ch, uint64_t level, uint64_t base
                                uint64_t *found, hipStream_t st)
 {
     if (count == 0) return 0;
-    dim3 g((unsigned)((count + p2_threads(8) - 1) / p2_threads(8)));
-    hipLaunchKernelGGL(k_p2_grind, g, dim3(p2_threads(8)), 0, st, ch[0], ch[1], ch[2], level, base, count,
+    const unsigned nt = p2_threads(8, count);
+    dim3 g((unsigned)((count + nt - 1) / nt));
+    hipLaunchKernelGGL(k_p2_grind, g, dim3(nt), 0, st, ch[0], ch[1], ch[2], level, base, count,
                        (unsigned long long *)found);
     return (int)hipGetLastError();
 }
@@ -810,7 +813,7 @@ extern "C" int p2_launch_leaves_carry(uint32_t width, const uint64_t *src, uint6
         }
         return (int)hipGetLastError();
     }
-    const unsigned nt = p2_threads(width);
+    const unsigned nt = p2_threads(width, nrows);
     dim3 g((unsigned)((nrows + nt - 1) / nt));
     switch (width) {
     case 8: hipLaunchKernelGGL(k_p2_leaves<8>, g, dim3(nt), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
@@ -837,7 +840,7 @@ extern "C" int p2_launch_tree_levels(uint32_t width, uint64_t *tree, uint64_t nl
             default: return -1;
             }
         } else {
-            const unsigned nt = p2_threads(width);
+            const unsigned nt = p2_threads(width, next);
             dim3 g((unsigned)((next + nt - 1) / nt));
             switch (width) {
             case 8: hipLaunchKernelGGL(k_p2_nodes<8>, g, dim3(nt), 0, st, tree, off, pending, pad, next); break;
@@ -862,7 +865,7 @@ extern "C" int p2_launch_mul_peak(const uint64_t *in, uint64_t *out, uint64_t la
 extern "C" int p2_launch_permute(uint32_t width, uint64_t *states, uint64_t count, hipStream_t st)
 {
     if (count == 0) return 0;
-    const unsigned nt = p2_threads(width);
+    const unsigned nt = p2_threads(width, count);
     dim3 g((unsigned)((count + nt - 1) / nt));
     switch (width) {
     case 8: hipLaunchKernelGGL(k_p2_permute_many<8>, g, dim3(nt), 0, st, states, count); break;
