@@ -264,7 +264,9 @@ __device__ __forceinline__ void gl_reducek3(const gl_prodk *x, uint64_t *out)
     for (int i = 0; i < 3; i++) out[i] = gl_pack(r0[i], r1[i]);
 }
 
-// One lane of gl_prodk3 / gl_reducek3, hazard gaps filled with s_nop.
+// One lane of gl_prodk3 / gl_reducek3, the gaps that no instruction fills taken by s_nop:
+// k is read three multiply-adds after its write, and scalar instructions wait for a mask
+// that a vector instruction writes by themselves.
 template <bool BU = false>
 __device__ __forceinline__ uint64_t gl_mulk1(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi)
 {
@@ -280,11 +282,9 @@ __device__ __forceinline__ uint64_t gl_mulk1(uint64_t a, uint64_t b, uint32_t s_
     uint64_t lo = gl_pack((uint32_t)p, (uint32_t)u), r, c, bm, m;
     asm("v_mad_u64_u32 %0, %1, %2, -1, %3" : "=&v"(r), "=&s"(c) : "v"((uint32_t)h), "v"(lo));
     uint32_t r0 = (uint32_t)r, r1 = (uint32_t)(r >> 32), tm, tn;
-    asm("s_nop 1\n\t"
-        "v_subb_co_u32_e64 %[r0], %[b], %[r0], %[x3], %[k]\n\t"
+    asm("v_subb_co_u32_e64 %[r0], %[b], %[r0], %[x3], %[k]\n\t"
         "s_nop 1\n\t"
         "v_subb_co_u32_e64 %[r1], %[b], %[r1], 0, %[b]\n\t"
-        "s_nop 1\n\t"
         "s_andn2_b64 %[m], %[c], %[b]\n\t"
         "s_andn2_b64 %[b], %[b], %[c]\n\t"
         "v_cndmask_b32_e64 %[tm], 0, -1, %[m]\n\t"
@@ -298,6 +298,59 @@ __device__ __forceinline__ uint64_t gl_mulk1(uint64_t a, uint64_t b, uint32_t s_
     return gl_pack(r0, r1);
 }
 
+// Two products of gl_mulk1 in step: the second one's instructions stand in the first
+// one's gaps (one wait state is left to s_nop).
+__device__ __forceinline__ void gl_mulk2(const uint64_t *a, const uint64_t *b, uint64_t *out)
+{
+    uint64_t p[2], t[2], u[2], k[2], h[2], r[2], c[2], bm[2], m[2];
+    uint32_t r0[2], r1[2], tm[2], tn[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        p[i] = (uint64_t)(uint32_t)a[i] * (uint32_t)b[i];
+        t[i] = (uint64_t)(uint32_t)a[i] * (uint32_t)(b[i] >> 32) + (p[i] >> 32);
+    }
+    asm("v_mad_u64_u32 %0, %2, %4, %6, %8\n\t"
+        "v_mad_u64_u32 %1, %3, %5, %7, %9"
+        : "=&v"(u[0]), "=&v"(u[1]), "=&s"(k[0]), "=&s"(k[1])
+        : "v"((uint32_t)(a[0] >> 32)), "v"((uint32_t)(a[1] >> 32)), "v"((uint32_t)b[0]), "v"((uint32_t)b[1]), "v"(t[0]),
+          "v"(t[1]));
+#pragma unroll
+    for (int i = 0; i < 2; i++) h[i] = (uint64_t)(uint32_t)(a[i] >> 32) * (uint32_t)(b[i] >> 32) + (u[i] >> 32);
+    asm("v_mad_u64_u32 %0, %2, %4, -1, %6\n\t"
+        "v_mad_u64_u32 %1, %3, %5, -1, %7"
+        : "=&v"(r[0]), "=&v"(r[1]), "=&s"(c[0]), "=&s"(c[1])
+        : "v"((uint32_t)h[0]), "v"((uint32_t)h[1]), "v"(gl_pack((uint32_t)p[0], (uint32_t)u[0])),
+          "v"(gl_pack((uint32_t)p[1], (uint32_t)u[1])));
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        r0[i] = (uint32_t)r[i];
+        r1[i] = (uint32_t)(r[i] >> 32);
+    }
+    asm("v_subb_co_u32_e64 %[r0a], %[ba], %[r0a], %[x3a], %[ka]\n\t"
+        "v_subb_co_u32_e64 %[r0b], %[bb], %[r0b], %[x3b], %[kb]\n\t"
+        "s_nop 0\n\t"
+        "v_subb_co_u32_e64 %[r1a], %[ba], %[r1a], 0, %[ba]\n\t"
+        "v_subb_co_u32_e64 %[r1b], %[bb], %[r1b], 0, %[bb]\n\t"
+        "s_andn2_b64 %[ma], %[ca], %[ba]\n\t"
+        "s_andn2_b64 %[ba], %[ba], %[ca]\n\t"
+        "s_andn2_b64 %[mb], %[cb], %[bb]\n\t"
+        "s_andn2_b64 %[bb], %[bb], %[cb]\n\t"
+        "v_cndmask_b32_e64 %[tma], 0, -1, %[ma]\n\t"
+        "v_cndmask_b32_e64 %[tmb], 0, -1, %[mb]\n\t"
+        "v_addc_co_u32_e64 %[r0a], %[ca], %[r0a], %[tma], %[ba]\n\t"
+        "v_addc_co_u32_e64 %[r0b], %[cb], %[r0b], %[tmb], %[bb]\n\t"
+        "v_cndmask_b32_e64 %[tma], 0, -1, %[ba]\n\t"
+        "v_cndmask_b32_e64 %[tmb], 0, -1, %[bb]\n\t"
+        "v_addc_co_u32_e64 %[r1a], %[ca], %[r1a], %[tma], %[ca]\n\t"
+        "v_addc_co_u32_e64 %[r1b], %[cb], %[r1b], %[tmb], %[cb]"
+        : [r0a] "+v"(r0[0]), [r0b] "+v"(r0[1]), [r1a] "+v"(r1[0]), [r1b] "+v"(r1[1]), [tma] "=&v"(tm[0]),
+          [tmb] "=&v"(tm[1]), [ba] "=&s"(bm[0]), [bb] "=&s"(bm[1]), [ma] "=&s"(m[0]), [mb] "=&s"(m[1]), [ca] "+s"(c[0]),
+          [cb] "+s"(c[1])
+        : [x3a] "v"((uint32_t)(h[0] >> 32)), [x3b] "v"((uint32_t)(h[1] >> 32)), [ka] "s"(k[0]), [kb] "s"(k[1])
+        : "scc");
+    out[0] = gl_pack(r0[0], r1[0]);
+    out[1] = gl_pack(r0[1], r1[1]);
+}
 
 // Three arbitrary 64-bit words to canonical form in place: r >= p exactly when
 // r + (2^32 - 1) carries out of 64 bits, and then that sum is r - p.

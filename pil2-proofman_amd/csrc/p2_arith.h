@@ -129,9 +129,7 @@ __device__ __forceinline__ uint64_t hz_fold(hz a)
     asm("v_add_co_u32_e64 %[r1], %[c], %[r1], %[h0]\n\t"
         "s_nop 1\n\t"
         "v_subb_co_u32_e64 %[r0], %[b], %[r0], 0, %[c]\n\t"
-        "s_nop 1\n\t"
         "s_andn2_b64 %[c], %[c], %[b]\n\t"
-        "s_nop 0\n\t"
         "v_addc_co_u32_e64 %[r1], %[b], %[r1], 0, %[c]"
         : [r0] "+v"(r0), [r1] "+v"(r1), [c] "=&s"(c), [b] "=&s"(b)
         : [h0] "v"((uint32_t)a.hi)
@@ -141,6 +139,9 @@ __device__ __forceinline__ uint64_t hz_fold(hz a)
 
 // a*b mod p as a 64-bit word (any 64-bit a, b)
 __device__ __forceinline__ uint64_t p2_mul(uint64_t a, uint64_t b) { return gl_mulk1(a, b, 0, 0); }
+
+// two of them in step
+__device__ __forceinline__ void p2_mul2(const uint64_t *a, const uint64_t *b, uint64_t *out) { gl_mulk2(a, b, out); }
 
 // a*b + s mod p as a 64-bit word (s = s_hi:s_lo)
 __device__ __forceinline__ uint64_t p2_mul_add(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi)
@@ -180,6 +181,7 @@ __device__ void hz_fold3(const hz *a, uint64_t *out);
 __device__ uint64_t hz_fold(hz a);
 __device__ uint64_t lz_fold(lz a);
 __device__ uint64_t p2_mul(uint64_t a, uint64_t b);
+__device__ void p2_mul2(const uint64_t *a, const uint64_t *b, uint64_t *out);
 __device__ uint64_t p2_mul_add(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi);
 __device__ uint64_t p2_mul_add_u(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi);
 

@@ -131,9 +131,18 @@ template <int W> struct Operands {
     }
 };
 
-// Per segment and out-word the constant of its result, as the two 64-bit addends of
-// the halves form: the correction for the signed bytes, the round constant added to
-// the word next, and 2^47 in each half, which makes the sums non-negative.
+// The constant v of a result as the two 64-bit addends of the halves form, with 2^47 in
+// each half, which makes the sums non-negative
+constexpr void addends(uint64_t v, uint64_t *k)
+{
+    const uint64_t bias = 1ULL << 47, off = add(bias, mul(bias, 1ULL << 32));
+    uint64_t d = add(v, GL_P - off);
+    k[0] = bias + (uint32_t)d;
+    k[1] = bias + (d >> 32);
+}
+
+// Per segment and out-word the addends of its result: the correction for the signed
+// bytes and the round constant added to the word next.
 template <int W> struct Addends {
     static constexpr int NOUT = Forms<W>::NOUT;
     uint64_t k[P2_SEGS][NOUT][2];
@@ -148,10 +157,7 @@ template <int W> struct Addends {
                 if (o < P2_SEG && r < P2_SEG * P2_SEGS) v = add(v, rc(W, 4 * W + r) % GL_P);
                 // after the last segment the first of the closing full rounds follows
                 if (o >= P2_SEG - 1 && g == P2_SEGS - 1) v = add(v, rc(W, 4 * W + 22 + o - (P2_SEG - 1)) % GL_P);
-                const uint64_t bias = 1ULL << 47, off = add(bias, mul(bias, 1ULL << 32));
-                uint64_t d = add(v, GL_P - off);
-                k[g][o][0] = bias + (uint32_t)d;
-                k[g][o][1] = bias + (d >> 32);
+                addends(v, k[g][o]);
             }
     }
 };

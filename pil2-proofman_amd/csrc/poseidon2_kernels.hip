@@ -119,13 +119,13 @@ __device__ __forceinline__ void ext_layer_hz(const uint64_t *s, hz *t)
 // x^7 (any 64-bit word in, congruent word out)
 __device__ __forceinline__ uint64_t pow7(uint64_t x)
 {
-    uint64_t x2 = p2_mul(x, x);
-    uint64_t x3 = p2_mul(x2, x);
-    uint64_t x4 = p2_mul(x2, x2);
-    return p2_mul(x3, x4);
+    uint64_t x2 = p2_mul(x, x), a[2] = {x2, x2}, b[2] = {x, x2}, z[2];
+    p2_mul2(a, b, z);
+    return p2_mul(z[0], z[1]);
 }
 
 #include "p2_partial.h"
+#include "p2_rows.h"
 
 // x^7 on three lanes, each product interleaved across the lanes
 __device__ __forceinline__ void pow7_3(const uint64_t *x, uint64_t *out)
@@ -407,184 +407,103 @@ __global__ __launch_bounds__(p2_max_threads(W), 4) void k_p2_nodes(uint64_t *__r
 }
 
 // ------------------------------------------------- cooperative levels ----
-// Upper tree levels have too few parents to fill the GPU with one permutation
-// per lane, so their time is the latency of one permutation. Here the 16 lanes
-// of a DPP row share one permutation: lane i holds state word i and lanes >= W
-// hold zero. Full rounds run all S-boxes at once; M4 reads the four words of
-// the lane's quad through DPP quad broadcasts; column sums and the state sum of
-// the partial rounds are DPP row rotations.
-
-// DPP reads of a VGPR need two wait states after its VALU write; values made by
-// inline asm pass through this barrier-nop first (the "+v" ties the order).
-__device__ __forceinline__ void dpp_ready(uint32_t &a, uint32_t &b, uint32_t &c)
-{
-    asm volatile("s_nop 1" : "+v"(a), "+v"(b), "+v"(c));
-}
-
-// the same barrier for two 64-bit values
-__device__ __forceinline__ void dpp_ready64(uint64_t &a, uint64_t &b)
-{
-    asm volatile("s_nop 1" : "+v"(a), "+v"(b));
-}
-
-template <int CTRL>
-__device__ __forceinline__ uint64_t dpp_u64(uint64_t v)
-{
-    uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)v, CTRL, 0xF, 0xF, false);
-    uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), CTRL, 0xF, 0xF, false);
-    return gl_pack(lo, hi);
-}
-
-constexpr int dpp_quad_bcast(int k) { return k | (k << 2) | (k << 4) | (k << 6); }
-constexpr int dpp_row_ror(int n) { return 0x120 + n; }
-
-__device__ __forceinline__ lz lz_add1(lz a, lz b)
-{
-    lz r;
-    lz_add_n<1>(&r, &a, &b);
-    return r;
-}
-
-// M_E on the row in halves form: the quad's four words are broadcast as 32-bit
-// halves, M4 runs on each half in 64-bit sums, and the column sum over the
-// blocks is two DPP row rotations of the 64-bit accumulators. Lane i gets
-// (M4 x_quad)[i mod 4] + its column sum; lanes >= W get zero.
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
-}
-
+// One tree level, 16 lanes per parent (p2_rows.h; same layout and pad rule as k_p2_nodes).
+// Bound by the latency of one permutation: about 3,600 instructions of a wave, most of
+// them 8 bytes long and 5.5 cycles apart when the wave has its SIMD to itself (11.5 us a
+// level at width 12, 10.4 in a fused launch; 18 us with DPP row sums and diagonal
+// products). Two waves a SIMD: at four the operands read ahead spill (116 against 108 us
+// for a tree of 8,192 leaves).
 template <int W>
-__device__ __forceinline__ hz ext_coop_hz(uint64_t x, uint32_t i, bool live)
+__global__ __launch_bounds__(P2_ROW_THREADS, 2) void k_p2_nodes_coop(uint64_t *__restrict__ tree, uint64_t in_off,
+                                                                     uint64_t pending, uint64_t pad, uint64_t nnext)
 {
-    uint64_t xv = x, dummy = 0;
-    dpp_ready64(xv, dummy);
-    uint32_t xl = (uint32_t)xv, xh = (uint32_t)(xv >> 32);
-    uint32_t q = i & 3;
-    uint64_t y[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        uint32_t v = h ? xh : xl;
-        uint64_t a0 = dpp_u32<dpp_quad_bcast(0)>(v), a1 = dpp_u32<dpp_quad_bcast(1)>(v);
-        uint64_t a2 = dpp_u32<dpp_quad_bcast(2)>(v), a3 = dpp_u32<dpp_quad_bcast(3)>(v);
-        uint64_t t0 = a0 + a1, t1 = a2 + a3;
-        uint64_t t2 = (a1 << 1) + t1, t3 = (a3 << 1) + t0;
-        uint64_t t4 = (t1 << 2) + t3, t5 = (t0 << 2) + t2;
-        y[h] = q == 0 ? t3 + t5 : q == 1 ? t5 : q == 2 ? t2 + t4 : t4;
-    }
-    hz c = {y[0], y[1]};
-    dpp_ready64(c.lo, c.hi);
-    c.lo += dpp_u64<dpp_row_ror(4)>(c.lo);
-    c.hi += dpp_u64<dpp_row_ror(4)>(c.hi);
-    dpp_ready64(c.lo, c.hi);
-    c.lo += dpp_u64<dpp_row_ror(8)>(c.lo);
-    c.hi += dpp_u64<dpp_row_ror(8)>(c.hi);
-    return live ? hz{y[0] + c.lo, y[1] + c.hi} : hz{0, 0};
-}
-
-template <int W>
-__device__ __forceinline__ uint64_t p2_permute_coop(uint64_t s, uint32_t i)
-{
-    const bool live = i < (uint32_t)W;
-    const uint32_t li = live ? i : 0;
-    hz t = ext_coop_hz<W>(s, i, live);
-#pragma unroll 1
-    for (int r = 0; r < 4; r++) {
-        uint64_t rc = live ? P2Tab<W>::rc(r * W + li) : 0;
-        t.lo += (uint32_t)rc;
-        t.hi += rc >> 32;
-        t = ext_coop_hz<W>(pow7(hz_fold(t)), i, live);
-    }
-    s = hz_fold(t);
-    const uint64_t d = live ? P2Tab<W>::d(li) : 0;
-#pragma unroll 1
-    for (int r = 0; r < 22; r++) {
-        uint64_t x0 = pow7(lz_fold(lz_add1(lz_of(s), lz_of(P2Tab<W>::rc(4 * W + r)))));
-        s = i == 0 ? x0 : s;
-        // row sum in halves form: the two 32-bit halves in 64-bit accumulators
-        // (below 16 * 2^32 after the four rotations), one 64-bit add per step
-        hz v = {(uint32_t)s, s >> 32};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            dpp_ready64(v.lo, v.hi);
-            switch (k) {
-            case 0: v.lo += dpp_u64<dpp_row_ror(1)>(v.lo); v.hi += dpp_u64<dpp_row_ror(1)>(v.hi); break;
-            case 1: v.lo += dpp_u64<dpp_row_ror(2)>(v.lo); v.hi += dpp_u64<dpp_row_ror(2)>(v.hi); break;
-            case 2: v.lo += dpp_u64<dpp_row_ror(4)>(v.lo); v.hi += dpp_u64<dpp_row_ror(4)>(v.hi); break;
-            default: v.lo += dpp_u64<dpp_row_ror(8)>(v.lo); v.hi += dpp_u64<dpp_row_ror(8)>(v.hi); break;
-            }
-        }
-        uint64_t sum = hz_fold(v);
-        s = live ? p2_mul_add(s, d, (uint32_t)sum, (uint32_t)(sum >> 32)) : 0;
-    }
-    t = {(uint32_t)s, s >> 32};
-#pragma unroll 1
-    for (int r = 0; r < 4; r++) {
-        uint64_t rc = live ? P2Tab<W>::rc(4 * W + 22 + r * W + li) : 0;
-        t.lo += (uint32_t)rc;
-        t.hi += rc >> 32;
-        t = ext_coop_hz<W>(pow7(hz_fold(t)), i, live);
-    }
-    return hz_fold(t);
-}
-
-// One tree level, 16 lanes per parent (same layout and pad rule as k_p2_nodes).
-template <int W>
-__global__ __launch_bounds__(P2_THREADS) void k_p2_nodes_coop(uint64_t *__restrict__ tree, uint64_t in_off,
-                                                              uint64_t pending, uint64_t pad, uint64_t nnext)
-{
-    constexpr int ARITY = W / 4;
-    uint64_t par = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    uint32_t i = threadIdx.x & 15;
-    bool active = par < nnext;  // whole rows are active or not
+    __shared__ p2_v4i ops[p2_row_pieces<W>()];
+    p2_row<W> row;
+    row.start(ops);
+    const uint64_t par = (uint64_t)blockIdx.x * (P2_ROW_THREADS / 16) + threadIdx.x / 64 * 4 + (threadIdx.x & 15) / 4;
+    const bool active = par < nnext;
     uint64_t s = 0;
-    if (active && i < (uint32_t)W && par * ARITY + (i >> 2) < pending) s = tree[in_off + par * W + i];
-    if (active && par == nnext - 1 && i == 0) {
+    if (active && row.word < (uint32_t)W && par * (W / 4) + row.q < pending) s = tree[in_off + par * W + row.word];
+    if (active && par == nnext - 1 && row.word == 0) {
         for (uint64_t z = 0; z < pad * 4; z++) tree[in_off + pending * 4 + z] = 0;
     }
-    s = p2_permute_coop<W>(s, i);
-    if (active && i < 4) tree[in_off + (pending + pad) * 4 + par * 4 + i] = gl_canon(s);
+    s = row.permute(s, true);
+    if (active && row.q == 0) tree[in_off + (pending + pad) * 4 + par * 4 + row.g] = gl_canon(s);
 }
 
-// Leaves of short trees, 16 lanes per row (same sponge as k_p2_leaves): lane i < RATE
-// absorbs column c0 + i, capacity lanes RATE..RATE+3 take the previous output words
-// 0..3 (a DPP row rotation by RATE), lanes >= W stay zero.
+// Up to p2_fused_levels(W / 4) levels in one launch: a block takes the children of 16
+// (arity 3: 9) parents and works its way up to one digest, through LDS, so that a level
+// costs its permutation without a launch and first loads of its own (arity 3, 8,192
+// leaves: 104.7 us in nine launches, 94.7 us in four; 163 us before the permutation ran
+// on the matrix cores). The block index is that of the last digest. Two waves a SIMD: with
+// one the compiler keeps the products' sums in AGPRs and copies them out (97.9 us).
+#define P2_FUSED_BLOCKS 256
+constexpr __host__ __device__ int p2_fused_levels(int arity) { return arity == 2 ? 5 : 3; }
+constexpr __host__ __device__ unsigned p2_fused_parents(int arity) { return arity == 3 ? 9 : 16; }
+
 template <int W>
-__global__ __launch_bounds__(P2_THREADS) void k_p2_leaves_coop(const uint64_t *__restrict__ src, uint64_t rs,
-                                                               uint64_t cs, uint64_t ncols, uint64_t nrows,
-                                                               uint64_t *__restrict__ out, uint32_t carry)
+__global__ __launch_bounds__(P2_ROW_THREADS, 2) void k_p2_levels(uint64_t *__restrict__ tree, uint64_t in_off,
+                                                                 uint64_t pending, int levels)
+{
+    constexpr uint64_t ARITY = W / 4;
+    __shared__ p2_v4i ops[p2_row_pieces<W>()];
+    __shared__ uint64_t digest[P2_ROW_THREADS / 16 * 4];
+    p2_row<W> row;
+    row.start(ops);
+    const uint32_t first = threadIdx.x / 64 * 4, slot = first + (threadIdx.x & 15) / 4;
+    uint32_t count = p2_fused_parents(ARITY);  // parents of this block at the level
+#pragma unroll 1
+    for (int k = 0; k < levels; k++, count /= ARITY) {
+        const uint64_t next = (pending + ARITY - 1) / ARITY, pad = next * ARITY - pending;
+        const uint64_t par = (uint64_t)blockIdx.x * count + slot;
+        const bool active = slot < count && par < next;
+        uint64_t s = 0;
+        if (active && row.word < (uint32_t)W && par * ARITY + row.q < pending)
+            s = k == 0 ? tree[in_off + par * W + row.word] : digest[(slot * ARITY + row.q) * 4 + row.g];
+        if (active && par == next - 1 && row.word == 0) {
+            for (uint64_t z = 0; z < pad * 4; z++) tree[in_off + pending * 4 + z] = 0;
+        }
+        if (k == 0 || first < count) s = gl_canon(row.permute(s, k == 0));
+        __syncthreads();  // every wave has read its children
+        in_off += next * W;
+        if (active && row.q == 0) {
+            digest[slot * 4 + row.g] = s;
+            tree[in_off + par * 4 + row.g] = s;
+        }
+        __syncthreads();
+        pending = next;
+    }
+}
+
+// Leaves of short trees, 16 lanes per row (same sponge as k_p2_leaves): the lane of rate
+// word w absorbs column c0 + w, the capacity lanes (q = W/4 - 1) take the previous output
+// words 0 .. 3 from the first lane of their quad.
+template <int W>
+__global__ __launch_bounds__(P2_ROW_THREADS, 2) void k_p2_leaves_coop(const uint64_t *__restrict__ src, uint64_t rs,
+                                                                      uint64_t cs, uint64_t ncols, uint64_t nrows,
+                                                                      uint64_t *__restrict__ out, uint32_t carry)
 {
     constexpr int RATE = W - 4;
-    uint64_t r = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-    uint32_t i = threadIdx.x & 15;
-    bool active = r < nrows;  // whole rows are active or not
+    __shared__ p2_v4i ops[p2_row_pieces<W>()];
+    p2_row<W> row;
+    const uint64_t r = (uint64_t)blockIdx.x * (P2_ROW_THREADS / 16) + threadIdx.x / 64 * 4 + (threadIdx.x & 15) / 4;
     if (ncols == 0) {
-        if (active && i < 4 && !carry) out[r * 4 + i] = 0;
+        row.start(ops);
+        if (r < nrows && row.q == 0 && !carry) out[r * 4 + row.g] = 0;
         return;
     }
-    const uint64_t *row = src + (active ? r : 0) * rs;
-    uint64_t s = 0;
+    row.start(ops);
+    row.stage();
+    const bool active = r < nrows;
+    const uint64_t *in = src + (active ? r : 0) * rs;
+    uint64_t s = active && carry && row.q == 0 ? out[r * 4 + row.g] : 0;
     for (uint64_t c0 = 0; c0 < ncols; c0 += RATE) {
-        uint64_t carried = 0;
-        if (c0 == 0 && carry && active && i >= (uint32_t)RATE && i < (uint32_t)W) {
-            carried = out[r * 4 + (i - RATE)];  // continued sponge (see k_p2_leaves)
-        } else if (c0 > 0) {  // capacity <- previous output words 0..3
-            uint32_t lo = (uint32_t)s, hi = (uint32_t)(s >> 32), z = 0;
-            dpp_ready(lo, hi, z);
-            lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)lo, dpp_row_ror(RATE), 0xF, 0xF, false);
-            hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)hi, dpp_row_ror(RATE), 0xF, 0xF, false);
-            carried = ((uint64_t)hi << 32) | lo;
-        }
-        uint64_t x = 0;
-        if (i < (uint32_t)RATE) {
-            if (active && c0 + i < ncols) x = row[(c0 + i) * cs];
-        } else if (i < (uint32_t)W) {
-            x = carried;
-        }
-        s = p2_permute_coop<W>(x, i);
+        asm volatile("s_nop 1" : "+v"(s));  // DPP reads two wait states after the write
+        uint64_t x = gl_pack((uint32_t)p2_dpp<0x00>((int)(uint32_t)s), (uint32_t)p2_dpp<0x00>((int)(s >> 32)));
+        if (row.word < (uint32_t)RATE) x = active && c0 + row.word < ncols ? in[(c0 + row.word) * cs] : 0;
+        s = row.permute(x, false);
     }
-    if (active && i < 4) out[r * 4 + i] = gl_canon(s);
+    if (active && row.q == 0) out[r * 4 + row.g] = gl_canon(s);
 }
 
 // ----------------------------------------------------------- grinding ----
@@ -804,11 +723,11 @@ extern "C" int p2_launch_leaves_carry(uint32_t width, const uint64_t *src, uint6
 {
     if (nrows == 0) return 0;
     if (nrows <= P2_COOP_LEAF_MAX_ROWS) {  // too few rows to fill the GPU: 16 lanes per row
-        dim3 g((unsigned)((nrows * 16 + P2_THREADS - 1) / P2_THREADS));
+        dim3 g((unsigned)((nrows * 16 + P2_ROW_THREADS - 1) / P2_ROW_THREADS));
         switch (width) {
-        case 8: hipLaunchKernelGGL(k_p2_leaves_coop<8>, g, dim3(P2_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
-        case 12: hipLaunchKernelGGL(k_p2_leaves_coop<12>, g, dim3(P2_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
-        case 16: hipLaunchKernelGGL(k_p2_leaves_coop<16>, g, dim3(P2_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
+        case 8: hipLaunchKernelGGL(k_p2_leaves_coop<8>, g, dim3(P2_ROW_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
+        case 12: hipLaunchKernelGGL(k_p2_leaves_coop<12>, g, dim3(P2_ROW_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
+        case 16: hipLaunchKernelGGL(k_p2_leaves_coop<16>, g, dim3(P2_ROW_THREADS), 0, st, src, rs, cs, ncols, nrows, out, carry); break;
         default: return -1;
         }
         return (int)hipGetLastError();
@@ -831,12 +750,34 @@ extern "C" int p2_launch_tree_levels(uint32_t width, uint64_t *tree, uint64_t nl
     while (pending > 1) {
         uint64_t pad = (arity - pending % arity) % arity;
         uint64_t next = (pending + arity - 1) / arity;
-        if (next <= coop_max) {  // latency-bound level: 16 lanes per parent
-            dim3 g((unsigned)((next * 16 + P2_THREADS - 1) / P2_THREADS));
+        // one block a CU: above that the waves that arity 3 leaves idle (9 parents in 16
+        // places) and the shrinking upper levels cost more than the launches
+        const uint64_t per = p2_fused_parents((int)arity);
+        if (next <= coop_max && next <= P2_FUSED_BLOCKS * per) {
+            int levels = 0;
+            uint64_t n = pending, in_off = off, blocks = (next + per - 1) / per;
+            while (levels < p2_fused_levels((int)arity) && n > 1) {
+                uint64_t up = (n + arity - 1) / arity;
+                off += up * arity * 4;
+                n = up;
+                levels++;
+            }
+            dim3 g((unsigned)blocks), b(P2_ROW_THREADS);
             switch (width) {
-            case 8: hipLaunchKernelGGL(k_p2_nodes_coop<8>, g, dim3(P2_THREADS), 0, st, tree, off, pending, pad, next); break;
-            case 12: hipLaunchKernelGGL(k_p2_nodes_coop<12>, g, dim3(P2_THREADS), 0, st, tree, off, pending, pad, next); break;
-            case 16: hipLaunchKernelGGL(k_p2_nodes_coop<16>, g, dim3(P2_THREADS), 0, st, tree, off, pending, pad, next); break;
+            case 8: hipLaunchKernelGGL(k_p2_levels<8>, g, b, 0, st, tree, in_off, pending, levels); break;
+            case 12: hipLaunchKernelGGL(k_p2_levels<12>, g, b, 0, st, tree, in_off, pending, levels); break;
+            case 16: hipLaunchKernelGGL(k_p2_levels<16>, g, b, 0, st, tree, in_off, pending, levels); break;
+            default: return -1;
+            }
+            pending = n;
+            continue;
+        }
+        if (next <= coop_max) {  // latency-bound level: 16 lanes per parent
+            dim3 g((unsigned)((next * 16 + P2_ROW_THREADS - 1) / P2_ROW_THREADS));
+            switch (width) {
+            case 8: hipLaunchKernelGGL(k_p2_nodes_coop<8>, g, dim3(P2_ROW_THREADS), 0, st, tree, off, pending, pad, next); break;
+            case 12: hipLaunchKernelGGL(k_p2_nodes_coop<12>, g, dim3(P2_ROW_THREADS), 0, st, tree, off, pending, pad, next); break;
+            case 16: hipLaunchKernelGGL(k_p2_nodes_coop<16>, g, dim3(P2_ROW_THREADS), 0, st, tree, off, pending, pad, next); break;
             default: return -1;
             }
         } else {

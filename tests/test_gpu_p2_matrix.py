@@ -36,3 +36,24 @@ def test_tall_tree_matches_oracle(pc, oracle, arity, rows, extra):
     t.merkelize()
     torch.cuda.synchronize()
     assert (pc.to_host(t.nodes) == oracle.merkletree(src, arity)).all()
+
+
+@pytest.mark.parametrize("arity", [2, 3, 4])
+@pytest.mark.parametrize("rows", [2, 3, 4, 5, 9, 10, 16, 17, 27, 28, 32, 33, 64, 65, 82, 145, 255, 257, 1025, 6913,
+                                  8193, 16384])
+def test_short_tree_matches_oracle(pc, oracle, arity, rows):
+    """Trees whose levels take 16 lanes a permutation and several levels a launch: one to
+    three blocks of every kind, partly filled ones, pads, and the switch to single levels;
+    one or two blocks of columns, boundary words in every other row."""
+    import torch
+    cols = 4 * arity - 4 + (rows % 3) - 1
+    rng = np.random.default_rng(rows * 5 + arity)
+    src = rng.integers(0, 2**64, (rows, cols), dtype=np.uint64)
+    edge = np.array(EDGE_WORDS, dtype=np.uint64)[rng.integers(0, len(EDGE_WORDS), (rows, cols))]
+    src[::2] = edge[::2]
+    t = pc.MerkleTreeGL(arity, 0, True, rows, cols, source=pc.to_device(src))
+    t.nodes = pc.empty(t.num_nodes)
+    t.nodes.fill_(-1)
+    t.merkelize()
+    torch.cuda.synchronize()
+    assert (pc.to_host(t.nodes) == oracle.merkletree(src, arity)).all()
