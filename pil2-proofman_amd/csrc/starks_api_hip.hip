@@ -1306,6 +1306,7 @@ static hipStream_t g_fri_capture = nullptr;
 // then run side by side instead of one after another; each is a chain of
 // latency-bound levels.
 static constexpr uint32_t kFriBranches = 4;
+static constexpr uint64_t kFriFusedBits = 17;
 static hipStream_t g_fri_side[kFriBranches];
 static std::vector<hipEvent_t> g_fri_fork;         // one per layer
 static hipEvent_t g_fri_join[kFriBranches];
@@ -1337,15 +1338,20 @@ static int64_t fri_enqueue(const uint64_t *d_pol, uint64_t *d_work, const uint64
     bool used[kFriBranches] = {};
     int64_t rc = 0;
     for (uint64_t s = 0; s < n && !rc; s++) {
+        // The fold writes a short layer's tree source itself: the next fold, in place, then
+        // waits for no transpose. A long layer's rows would be written in pieces of 24 bytes.
+        const bool fused = s > 0 && s + 1 < n && steps[s] <= kFriFusedBits;
         if (s > 0) {
             int e = fri_launch_fold2(d_work, s == 1 ? d_pol : d_work, nullptr, d_ch + 3 * s, nbe, steps[s - 1],
-                                     steps[s], fri_tables(st), st);
+                                     steps[s], fri_tables(st), fused ? d_sources[s] : nullptr,
+                                     fused ? steps[s + 1] : 0, st);
             if (e) rc = fail(-100 - e, "fold launch failed");
         }
         if (!rc && s + 1 < n) {
             uint64_t rows = 1ull << steps[s + 1], cols = 3ull << (steps[s] - steps[s + 1]);
-            int e = fri_launch_transpose(d_sources[s], s == 0 ? d_pol : d_work, 1ull << steps[s],
-                                         (uint32_t)steps[s + 1], st);
+            int e = fused ? 0
+                          : fri_launch_transpose(d_sources[s], s == 0 ? d_pol : d_work, 1ull << steps[s],
+                                                 (uint32_t)steps[s + 1], st);
             hipStream_t ts = st;
             if (!e && branches) {
                 uint32_t b = (uint32_t)(s % kFriBranches);
