@@ -234,10 +234,9 @@ def _leaf_roofline(width, perms, leaf_ms, leaf_bytes, traffic, launches):
 
 
 def _lde_kernels(nb, nbe, cols):
-    """The four kernels of one LDE as the library launches them for this shape
-    (blowup 4 with two or more columns takes the two-column block kernel)."""
-    block = "k_lde_block2" if nbe - nb == 2 and cols >= 2 else "k_lde_block<false, false, false>"
-    return ("k_transpose_rm2cm", "k_ntt_strided_inv<false>", block, "k_ntt_strided_fwd<false, false>")
+    """The four kernels of one LDE (their names up to the shape's parameters)."""
+    return ("k_transpose_rm2cm", "k_ntt_strided_inv_mx<", "k_lde_block_mx<false, false, %d, " % (nbe - nb),
+            "k_ntt_strided_fwd_mx<false, ")
 # single-rate VALU instructions of one radix-2 butterfly at the floor: a reduced
 # Goldilocks product (4 v_mad_u64_u32 + a 7-instruction reduction) plus a 6-instruction
 # add and a 6-instruction sub
@@ -923,13 +922,16 @@ def _plain_from_host(args, pc, trace, lde, nodes, scratch, root, nb, nbe, cols, 
 
 
 def _profile_kernel(kernel, config):
-    """Per-launch counters of `kernel` from the committed rocprofv3 summary, or {}."""
+    """Per-launch counters of `kernel` (a name, or the beginning of exactly one) from
+    the committed rocprofv3 summary, or {}."""
     path = os.path.join(ROOT, "profiles", "traffic_%s.json" % config)
     try:
         with open(path) as f:
-            return json.load(f)["kernels"][kernel]
+            kernels = json.load(f)["kernels"]
     except (OSError, KeyError, ValueError):
         return {}
+    found = [k for k in kernels if k == kernel] or [k for k in kernels if k.startswith(kernel)]
+    return kernels[found[0]] if len(found) == 1 else {}
 
 
 def _profile_traffic(kernel, config):

@@ -384,6 +384,34 @@ __device__ __forceinline__ void gl_canon3(uint64_t *v)
     for (int k = 0; k < 3; k++) v[k] = gl_pack(s0[k], s1[k]);
 }
 
+// Two of them
+__device__ __forceinline__ void gl_canon2(uint64_t *v)
+{
+    uint32_t s0[2], s1[2], t0[2], t1[2];
+    uint64_t K[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        s0[k] = (uint32_t)v[k];
+        s1[k] = (uint32_t)(v[k] >> 32);
+    }
+    asm("v_add_co_u32_e64 %[t0a], %[Ka], -1, %[s0a]\n\t"
+        "v_add_co_u32_e64 %[t0b], %[Kb], -1, %[s0b]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32_e64 %[t1a], %[Ka], 0, %[s1a], %[Ka]\n\t"
+        "v_addc_co_u32_e64 %[t1b], %[Kb], 0, %[s1b], %[Kb]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32_e64 %[s0a], %[s0a], %[t0a], %[Ka]\n\t"
+        "v_cndmask_b32_e64 %[s0b], %[s0b], %[t0b], %[Kb]\n\t"
+        "v_cndmask_b32_e64 %[s1a], %[s1a], %[t1a], %[Ka]\n\t"
+        "v_cndmask_b32_e64 %[s1b], %[s1b], %[t1b], %[Kb]"
+        : [s0a] "+v"(s0[0]), [s1a] "+v"(s1[0]), [t0a] "=&v"(t0[0]), [t1a] "=&v"(t1[0]), [Ka] "=&s"(K[0]),
+          [s0b] "+v"(s0[1]), [s1b] "+v"(s1[1]), [t0b] "=&v"(t0[1]), [t1b] "=&v"(t1[1]), [Kb] "=&s"(K[1])
+        :
+        : "scc");
+#pragma unroll
+    for (int k = 0; k < 2; k++) v[k] = gl_pack(s0[k], s1[k]);
+}
+
 template <int N> __device__ __forceinline__ void gl_add_n(uint64_t *out, const uint64_t *a, const uint64_t *b);
 template <int N> __device__ __forceinline__ void gl_sub_n(uint64_t *out, const uint64_t *a, const uint64_t *b);
 template <int N> __device__ __forceinline__ void gl_prod_reduce_canon_n(uint64_t *out, const gl_prod *x);
@@ -1129,6 +1157,8 @@ __device__ __forceinline__ uint64_t gl_mul_pow2(uint64_t x)
 }
 
 #else  // host pass: declarations only (kernels are compiled for the device)
+__device__ void gl_mulk2(const uint64_t *a, const uint64_t *b, uint64_t *out);
+__device__ void gl_canon2(uint64_t *v);
 template <int N> __device__ void gl_add_v(uint64_t *out, const uint64_t *a, const uint64_t *b);
 template <int N> __device__ void gl_sub_v(uint64_t *out, const uint64_t *a, const uint64_t *b);
 template <int N> __device__ void gl_mul_v(uint64_t *out, const uint64_t *a, const uint64_t *b);

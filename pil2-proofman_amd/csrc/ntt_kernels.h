@@ -23,7 +23,8 @@ struct NttTablesHost {
 };
 
 // LDE launch plan: the largest block tile (log2 values, <= 14; a shape that needs a
-// larger one gets it) and the most index bits per in-tile round (radix 2^radix_log).
+// larger one gets it) and the most index bits per in-tile round (radix 2^radix_log), for
+// the shapes whose rounds are on the VALU; those on the matrix cores have one plan.
 struct NttPlan {
     uint32_t tile_log, radix_log;
 };

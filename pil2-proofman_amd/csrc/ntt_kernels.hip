@@ -20,10 +20,11 @@
 //   pass 3  strided NTT: n1-point DIT over m (stride n2*B) -> natural order
 //
 // Inside a tile every sub-transform of 2^L points runs as rounds of at most 4
-// index bits (four-step again): a 2^r-point DFT in registers whose internal
-// twiddles are powers of w_16, and one twiddle per element between rounds,
+// index bits (four-step again): a 2^r-point DFT, on the matrix cores (ntt_matrix.h,
+// the shapes of mx_split) or in registers with internal twiddles that are powers of
+// w_16, and one twiddle per element between rounds,
 // w_{2^(q+r)}^(o*bitrev(j)) (o = the element's index bits below the round).
-// Each thread keeps 16 values per round; rounds exchange through LDS. The first
+// On the VALU each thread keeps 16 values per round; rounds exchange through LDS. The first
 // round of a pass reads global memory and the last one writes it, both in runs
 // of >= 64 bytes (whole 128-byte lines per XCD; see strided_tile).
 #include <algorithm>
@@ -530,10 +531,7 @@ __device__ __forceinline__ void line_load_b(uint64_t *__restrict__ s, const uint
 // Phase 1: the n2 values are loaded into LDS, then DIF rounds run with V = 16/B
 // values per thread (so every thread works); the last round scales the
 // coefficient at position k (index e = bitrev_{L1+L2}(m*n2 + k)) by 7^e / N.
-// LINES = 2: two lines of n2 values sit one after the other in LDS (line index at
-// bit L2 of the position) and the rounds run over both; a round's bits and twiddles
-// are those of the position within its line.
-template <int R, int V, int LINES = 1>
+template <int R, int V>
 __device__ __forceinline__ void block_dif_round(uint64_t *__restrict__ s, uint32_t q, bool last, uint32_t m,
                                                 uint32_t L2, uint32_t log_n, uint64_t n_inv, const NttTables &tb)
 {
@@ -542,7 +540,7 @@ __device__ __forceinline__ void block_dif_round(uint64_t *__restrict__ s, uint32
     uint32_t t = threadIdx.x;
 #pragma unroll
     for (int gg = 0; gg < G; gg++) {
-        RoundPos p = round_pos(gg * (((uint32_t)LINES << L2) >> Log2<V>::v) + t, 0, q);
+        RoundPos p = round_pos(gg * ((1u << L2) >> Log2<V>::v) + t, 0, q);
         uint64_t *sb = s + lds_addr(round_m(p, 0, q, LR));
         uint64_t v[R];
 #pragma unroll
@@ -558,7 +556,7 @@ __device__ __forceinline__ void block_dif_round(uint64_t *__restrict__ s, uint32
             uint64_t lo[R], hi[R], ni[R];
 #pragma unroll
             for (int j = 0; j < R; j++) {
-                uint32_t e = bitrev32((m << L2) | (round_m(p, j, q, LR) & ((1u << L2) - 1)), log_n);
+                uint32_t e = bitrev32((m << L2) | (round_m(p, j, q, LR)), log_n);
                 lo[j] = tb.shl[tw_lo(e, tb)];
                 hi[j] = tb.shh[tw_hi(e, tb)];
                 ni[j] = n_inv;
@@ -572,12 +570,12 @@ __device__ __forceinline__ void block_dif_round(uint64_t *__restrict__ s, uint32
     }
 }
 
-template <int V, int LINES = 1>
+template <int V>
 __device__ __forceinline__ void block_phase1(uint64_t *__restrict__ s, uint32_t m, uint32_t L2, uint32_t log_n,
                                              uint64_t n_inv, const NttTables &tb, bool scale, uint32_t rmax)
 {
     constexpr int LV = Log2<V>::v;
-    bool active = threadIdx.x < (((uint32_t)LINES << L2) >> LV);
+    bool active = threadIdx.x < ((1u << L2) >> LV);
     int rm = LV < (int)rmax ? LV : (int)rmax;
     int q = (int)L2;
     while (q > 0) {
@@ -586,10 +584,10 @@ __device__ __forceinline__ void block_phase1(uint64_t *__restrict__ s, uint32_t 
         bool last = (q == 0) && scale;
         if (active) {
             switch (r) {
-            case 4: if constexpr (V >= 16) block_dif_round<16, V, LINES>(s, q, last, m, L2, log_n, n_inv, tb); break;
-            case 3: if constexpr (V >= 8) block_dif_round<8, V, LINES>(s, q, last, m, L2, log_n, n_inv, tb); break;
-            case 2: if constexpr (V >= 4) block_dif_round<4, V, LINES>(s, q, last, m, L2, log_n, n_inv, tb); break;
-            default: block_dif_round<2, V, LINES>(s, q, last, m, L2, log_n, n_inv, tb); break;
+            case 4: if constexpr (V >= 16) block_dif_round<16, V>(s, q, last, m, L2, log_n, n_inv, tb); break;
+            case 3: if constexpr (V >= 8) block_dif_round<8, V>(s, q, last, m, L2, log_n, n_inv, tb); break;
+            case 2: if constexpr (V >= 4) block_dif_round<4, V>(s, q, last, m, L2, log_n, n_inv, tb); break;
+            default: block_dif_round<2, V>(s, q, last, m, L2, log_n, n_inv, tb); break;
             }
         }
         __syncthreads();
@@ -719,67 +717,41 @@ __global__ __launch_bounds__(NTT_THREADS) void k_lde_block(const uint64_t *__res
     }
 }
 
-// The fused block pass for blowup 4 on two columns at once: block (m, c) takes line
-// m of columns 2c and 2c + 1. Phase 1 runs on both lines together (8 values per
-// thread instead of 4: radix-8 rounds, so half the rounds and barriers per line,
-// every thread busy). Phase 2 needs the whole tile for one line, so it runs on
-// the first line while each thread keeps four of the second line's coefficients
-// in registers; they go back to LDS for the second line's phase 2.
-__global__ __launch_bounds__(NTT_THREADS) void k_lde_block2(const uint64_t *__restrict__ in, uint64_t cs_in,
-                                                            uint64_t *__restrict__ out, uint64_t cs_out, uint32_t L1,
-                                                            uint32_t L2, uint64_t n_inv, uint32_t rmax, NttTables tb)
+#include "ntt_matrix.h"
+
+typedef void (*MxStridedKernel)(uint64_t *, MxStrided, NttTables);
+typedef void (*MxBlockKernel)(const uint64_t *, uint64_t *, MxBlock, NttTables);
+
+static MxStridedKernel strided_inv_mx(uint32_t L1)
 {
-    constexpr uint32_t logb = 2;
-    extern __shared__ uint64_t s[];
-    const uint32_t m = blockIdx.x, n2 = 1u << L2, t = threadIdx.x, nt = blockDim.x;  // n2 = 4 * nt
-    const uint64_t c0 = 2ull * blockIdx.y;
-    const uint64_t *src = in + c0 * cs_in + ((uint64_t)m << L2);
-    {
-        uint64_t v[8];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            v[i] = __builtin_nontemporal_load(&src[t + i * nt]);
-            v[4 + i] = __builtin_nontemporal_load(&src[cs_in + t + i * nt]);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            s[lds_addr(t + i * nt)] = gl_canon(v[i]);
-            s[lds_addr(n2 + t + i * nt)] = gl_canon(v[4 + i]);
-        }
-    }
-    __syncthreads();
-    uint32_t log_n = L1 + L2;
-    block_phase1<8, 2>(s, m, L2, log_n, n_inv, tb, true, rmax);
-    uint64_t keep[4];  // the second line's coefficients during the first line's phase 2
-#pragma unroll
-    for (int i = 0; i < 4; i++) keep[i] = s[lds_addr(n2 + t + i * nt)];
-    __syncthreads();
-    uint32_t e1 = bitrev32(m, L1);
-    uint32_t shift_e = 2 * tb.bits - (log_n + logb);
-    uint32_t top = L2 + logb;
-    for (int line = 0; line < 2; line++) {
-        if (line == 1) {
-            __syncthreads();  // every thread has read the first line's last round from LDS
-#pragma unroll
-            for (int i = 0; i < 4; i++) s[lds_addr(t + i * nt)] = keep[i];
-            __syncthreads();
-        }
-        uint64_t *dst = out + (c0 + line) * cs_out + ((uint64_t)m << top);
-        uint32_t qq = logb;
-        bool first = true;
-        while (qq < top) {
-            uint32_t r = (top - qq) >= rmax ? rmax : (top - qq);
-            bool last = (qq + r == top);
-            switch (r) {
-            case 4: block_dit_round<16, false, false>(s, dst, qq, logb, first, last, e1, shift_e, L1, tb); break;
-            case 3: block_dit_round<8, false, false>(s, dst, qq, logb, first, last, e1, shift_e, L1, tb); break;
-            case 2: block_dit_round<4, false, false>(s, dst, qq, logb, first, last, e1, shift_e, L1, tb); break;
-            default: block_dit_round<2, false, false>(s, dst, qq, logb, first, last, e1, shift_e, L1, tb); break;
-            }
-            if (!last) __syncthreads();
-            first = false;
-            qq += r;
-        }
+    static const MxStridedKernel k[] = {k_ntt_strided_inv_mx<4>, k_ntt_strided_inv_mx<5>, k_ntt_strided_inv_mx<6>,
+                                        k_ntt_strided_inv_mx<7>, k_ntt_strided_inv_mx<8>, k_ntt_strided_inv_mx<9>,
+                                        k_ntt_strided_inv_mx<10>};
+    return k[L1 - 4];
+}
+template <bool INV> static MxStridedKernel strided_fwd_mx(uint32_t L1)
+{
+    static const MxStridedKernel k[] = {k_ntt_strided_fwd_mx<INV, 4>, k_ntt_strided_fwd_mx<INV, 5>,
+                                        k_ntt_strided_fwd_mx<INV, 6>, k_ntt_strided_fwd_mx<INV, 7>,
+                                        k_ntt_strided_fwd_mx<INV, 8>, k_ntt_strided_fwd_mx<INV, 9>,
+                                        k_ntt_strided_fwd_mx<INV, 10>};
+    return k[L1 - 4];
+}
+template <bool COEF_IN, bool INV, int LOGB> static MxBlockKernel block_mx_r(uint32_t r)
+{
+    static const MxBlockKernel k[] = {k_lde_block_mx<COEF_IN, INV, LOGB, 1>, k_lde_block_mx<COEF_IN, INV, LOGB, 2>,
+                                      k_lde_block_mx<COEF_IN, INV, LOGB, 3>, k_lde_block_mx<COEF_IN, INV, LOGB, 4>};
+    return k[r - 1];
+}
+// r: bits of the short round; INV: without blowup
+template <bool COEF_IN, bool INV> static MxBlockKernel block_mx(uint32_t log_b, uint32_t r)
+{
+    if constexpr (INV) return block_mx_r<COEF_IN, true, 0>(r);
+    switch (log_b) {
+    case 0: return block_mx_r<COEF_IN, false, 0>(r);
+    case 1: return block_mx_r<COEF_IN, false, 1>(r);
+    case 2: return block_mx_r<COEF_IN, false, 2>(r);
+    default: return block_mx_r<COEF_IN, false, 3>(r);
     }
 }
 
@@ -975,7 +947,20 @@ extern "C" int ntt_init_device(void)
             if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void *)k_q_block_inv, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        const void *blocks[] = {(const void *)k_lde_block2, (const void *)k_lde_block<false, false, false>,
+        for (uint32_t l1 = 4; l1 <= NTT_MAX_STRIDED; l1++) {
+            const void *strided[] = {(const void *)strided_inv_mx(l1), (const void *)strided_fwd_mx<false>(l1),
+                                     (const void *)strided_fwd_mx<true>(l1)};
+            for (const void *f : strided)
+                if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        }
+        for (uint32_t b = 0; b < 4; b++)
+            for (uint32_t r = 1; r <= 4; r++) {
+                const void *block[] = {(const void *)block_mx<false, false>(b, r), (const void *)block_mx<true, false>(b, r),
+                                       (const void *)block_mx<true, true>(0, r)};
+                for (const void *f : block)
+                    if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+            }
+        const void *blocks[] = {(const void *)k_lde_block<false, false, false>,
                                 (const void *)k_lde_block<false, false, true>,
                                 (const void *)k_lde_block<true, false, false>,
                                 (const void *)k_lde_block<true, false, true>,
@@ -1063,25 +1048,83 @@ static void launch_strided_fwd(uint64_t *data, uint64_t cs, uint32_t L1, uint32_
     }
 }
 
+// The split of a transform whose rounds run on the matrix cores (ntt_matrix.h): no strided
+// pass where a block holds a column, else the fewest rounds of four bits and then (L1 <= 8)
+// the smallest block of at least 2^11 values, several of which share a CU (2^18 x 75 to 2^20:
+// block and strided passes 919 us as 8 + 10 bits, 947 as 6 + 12). Returns false for
+// the shapes that keep the rounds on the VALU: lines of fewer than 2^8 coefficients, blocks
+// of fewer than 2^10 values (a wave), more than 8 copies of a coefficient (a piece holds them all),
+// transforms beyond 2^24 values.
+static bool mx_split(uint32_t log_n, uint32_t log_b, uint32_t *L1, uint32_t *L2)
+{
+    uint32_t best = ~0u;
+    if (log_b > 3) return false;
+    for (uint32_t l1 = log_n + log_b <= NTT_LOG_TILE ? 0 : 4; l1 <= NTT_MAX_STRIDED && l1 + 8 <= log_n; l1++) {
+        const uint32_t l2 = log_n - l1, tile = l2 + log_b, rounds = (l1 + 3) / 4 + (l2 + 3) / 4;
+        if (tile > NTT_LOG_TILE || tile < 10) continue;
+        if (rounds > best || (rounds == best && (l1 > 8 || tile < 11))) continue;
+        best = rounds;
+        *L1 = l1;
+        *L2 = l2;
+        if (l1 == 0) break;
+    }
+    return best != ~0u;
+}
+
+// Two columns a block of blowup 4 or 8 (all waves have work in phase 1) pay only where a
+// block has a CU to itself and there are 16 of them for each: 2^22 x 16 to 2^24 4.03 ms
+// instead of 4.12, but 2^16 x 100 to 2^18 365 us instead of 347, and 2^13 x 8 62 instead of 29.
+#define MX_PAIRS 8192
+// Strided tiles: four blocks of 256 threads a CU (2^18 x 75 forward 272 us; 292 with two of
+// 512 and 293 with eight of 128) while that leaves runs of whole 128-byte lines
+#define MX_STRIDED_TILE(L1) ((L1) <= 8 ? 12 : 13)
+#define MX_STRIDED_BLOCKS 1024  // of the launches that go on to further tiles
+
+static void launch_strided_mx(MxStridedKernel (*kernel)(uint32_t), uint64_t *data, uint64_t cs, uint32_t L1,
+                              uint32_t log_n2, uint64_t ncols, const NttTables &tb, hipStream_t st)
+{
+    if (!L1) return;
+    const uint32_t lt = strided_lt(L1, log_n2, MX_STRIDED_TILE(L1)), tiles = (uint32_t)ncols << (log_n2 - lt);
+    const MxStrided p = {cs, L1, log_n2, lt, log_n2 - lt, tiles};
+    hipLaunchKernelGGL(kernel(L1), dim3(L1 > 4 ? tiles : std::min<uint32_t>(tiles, MX_STRIDED_BLOCKS)), dim3(1u << (L1 + lt - MX_LOG_THREAD)),
+                       L1 > 4 ? lds_bytes(L1 + lt) : 0, st, data, p, tb);
+}
+
+template <bool COEF_IN, bool INV>
+static void launch_block_mx(const uint64_t *in, uint64_t cs_in, uint64_t *out, uint64_t cs_out, uint32_t L1, uint32_t L2,
+                            uint32_t log_b, uint64_t ncols, const NttTables &tb, hipStream_t st)
+{
+    const uint32_t per = !COEF_IN && log_b >= 2 && L2 + log_b == NTT_LOG_TILE && (ncols << L1) >= MX_PAIRS ? 2 : 1;
+    const MxBlock p = {cs_in, cs_out, ncols, L1, L2, per};
+    const size_t lds = lds_bytes(L2 + log_b);
+    dim3 g(1u << L1, (unsigned)((ncols + per - 1) / per)), b(1u << (L2 + log_b - MX_LOG_THREAD));
+    hipLaunchKernelGGL((block_mx<COEF_IN, INV>(log_b, (L2 - 1) % 4 + 1)), g, b, lds, st, in, out, p, tb);
+}
+
 // Launch geometry of an LDE of 2^log_n -> 2^log_ext rows under a plan: n2 * B <=
 // 2^tile values per block (tile <= 14), n1 = N / n2 <= 2^10 for one strided launch;
 // a shape that needs n1 > 2^10 at the requested tile gets the smallest tile that
 // fits, and beyond 2^14 values per block the strided passes take two launches
 // (n1 <= 2^20). Returns nonzero for a shape no plan covers (log_n >= 4 assumed).
 struct LdeGeometry {
-    uint32_t tile, rmax, L1, L2, lt_inv, lt_fwd;
+    uint32_t tile, rmax, L1, L2, lt_inv, lt_fwd;  // rmax 0: rounds on the matrix cores
 };
 static int lde_geometry(uint32_t log_n, uint32_t log_ext, const NttPlan *plan, LdeGeometry *g)
 {
     uint32_t log_b = log_ext - log_n;
+    uint32_t L1, L2;
+    if (mx_split(log_n, log_b, &L1, &L2)) {
+        *g = {0, 0, L1, L2, 0, 0};
+        return 0;
+    }
     uint32_t tile = plan ? plan->tile_log : NTT_LOG_TILE, rmax = plan ? plan->radix_log : 4;
     if (tile > NTT_LOG_TILE) tile = NTT_LOG_TILE;
     if (tile < log_b + 4) tile = log_b + 4;
     if (rmax < 1 || rmax > 4) rmax = 4;
-    uint32_t L2 = log_n;
+    L2 = log_n;
     if (L2 + log_b > tile) L2 = tile - log_b;
     if (log_n - L2 > NTT_MAX_STRIDED) L2 = std::min(log_n - NTT_MAX_STRIDED, (uint32_t)NTT_LOG_TILE - log_b);
-    uint32_t L1 = log_n - L2;
+    L1 = log_n - L2;
     if (L2 + log_b > NTT_LOG_TILE || L2 < 4 || L1 > 2 * NTT_MAX_STRIDED) return -2;  // n2*B <= 2^14, >= 16 values
     StridedPart pi[2], pf[2];
     strided_parts(L1, L2, tile, true, pi);
@@ -1126,6 +1169,15 @@ extern "C" int ntt_launch_lde(uint64_t *lde, const uint64_t *trace, uint64_t *sc
     LdeGeometry geo;
     if (lde_geometry(log_n, log_ext, plan, &geo)) return -2;
     uint32_t rmax = geo.rmax, L1 = geo.L1, L2 = geo.L2;
+    if (rmax == 0) {
+        launch_strided_mx(strided_inv_mx, scratch, N, L1, L2, ncols, tb, st);
+        if (ev) (void)hipEventRecord(ev[1], st);
+        launch_block_mx<false, false>(scratch, N, lde, N << log_b, L1, L2, log_b, ncols, tb, st);
+        if (ev) (void)hipEventRecord(ev[2], st);
+        launch_strided_mx(strided_fwd_mx<false>, lde, N << log_b, L1, L2 + log_b, ncols, tb, st);
+        if (ev) (void)hipEventRecord(ev[3], st);
+        return (int)hipGetLastError();
+    }
 
     // 1. strided inverse DIF over n1
     launch_strided_inv(scratch, N, L1, L2, geo.tile, ncols, tb, st);
@@ -1137,15 +1189,6 @@ extern "C" int ntt_launch_lde(uint64_t *lde, const uint64_t *trace, uint64_t *sc
         if (L1 > NTT_MAX_STRIDED) {
             hipLaunchKernelGGL((k_lde_block<false, false, true>), g, dim3(1u << (log_tile - 4)), lds_bytes(log_tile),
                                st, scratch, N, lde, N << log_b, L1, L2, log_b, n_inv, rmax, tb);
-        } else if (log_b == 2 && ncols >= 2) {
-            // column pairs two lines per block; an odd last column on its own
-            dim3 g2((unsigned)(1u << L1), (unsigned)(ncols / 2));
-            hipLaunchKernelGGL(k_lde_block2, g2, dim3(1u << (log_tile - 4)), lds_bytes(log_tile), st, scratch, N, lde,
-                               N << log_b, L1, L2, n_inv, rmax, tb);
-            if (ncols & 1)
-                hipLaunchKernelGGL((k_lde_block<false, false, false>), dim3((unsigned)(1u << L1), 1u),
-                                   dim3(1u << (log_tile - 4)), lds_bytes(log_tile), st, scratch + (ncols - 1) * N, N,
-                                   lde + (ncols - 1) * (N << log_b), N << log_b, L1, L2, log_b, n_inv, rmax, tb);
         } else {
             hipLaunchKernelGGL((k_lde_block<false, false, false>), g, dim3(1u << (log_tile - 4)), lds_bytes(log_tile),
                                st, scratch, N, lde, N << log_b, L1, L2, log_b, n_inv, rmax, tb);
@@ -1180,8 +1223,11 @@ extern "C" int ntt_launch_compute_q(uint64_t *cmq, const uint64_t *q, uint64_t q
     // the LDE's split: n2*B <= 2^14 values per block, n1 = N / n2 <= 2^10
     uint32_t L2 = log_n;
     if (L2 + log_b > NTT_LOG_TILE) L2 = NTT_LOG_TILE - log_b;
-    uint32_t L1 = log_n - L2, lb = L2 + log_b;
+    uint32_t L1 = log_n - L2;
+    const bool mx = mx_split(log_n, log_b, &L1, &L2);
+    uint32_t lb = L2 + log_b;
     if (L1 > 2 * NTT_MAX_STRIDED || L2 < 1 || lb < 4) return -2;
+    if (mx) n_inv_ext = gl_inv(1ull << lb);  // the strided pass scales by 2^-L1
 
     // 0. the q columns, column-major, into the last qDim columns of cmQ (consumed
     //    before the extension writes there)
@@ -1194,11 +1240,19 @@ extern "C" int ntt_launch_compute_q(uint64_t *cmq, const uint64_t *q, uint64_t q
         hipLaunchKernelGGL(k_transpose_rm2cm, tg, dim3(256), 0, st, q, qc, NExt, (uint64_t)q_dim, q_rs, NExt);
     }
     // 1. strided inverse DIF over n1 (stride n2*B)
-    launch_strided_inv(qc, NExt, L1, lb, NTT_STRIDED_TILE, q_dim, tb, st);
+    if (mx)
+        launch_strided_mx(strided_inv_mx, qc, NExt, L1, lb, q_dim, tb, st);
+    else
+        launch_strided_inv(qc, NExt, L1, lb, NTT_STRIDED_TILE, q_dim, tb, st);
     // 2a. inverse blocks -> scaled coefficient lines (coef: column c at coef + c*N)
     hipLaunchKernelGGL(k_q_block_inv, dim3(1u << L1, q_dim), dim3(1u << (lb - 4)), lds_bytes(lb), st, qc, NExt, coef,
                        N, L1, L2, log_b, q_deg, q_dim, n_inv_ext, shift_in, tb);
     // 2b. extension blocks (spread, DIT, twiddle) into cmQ
+    if (mx) {
+        launch_block_mx<true, false>(coef, N, cmq, NExt, L1, L2, log_b, ncols, tb, st);
+        launch_strided_mx(strided_fwd_mx<false>, cmq, NExt, L1, lb, ncols, tb, st);
+        return (int)hipGetLastError();
+    }
     if (L1 > NTT_MAX_STRIDED)
         hipLaunchKernelGGL((k_lde_block<true, false, true>), dim3(1u << L1, ncols), dim3(1u << (lb - 4)), lds_bytes(lb),
                            st, coef, N, cmq, NExt, L1, L2, log_b, (uint64_t)0, 4u, tb);
@@ -1240,6 +1294,16 @@ extern "C" int ntt_launch_ntt(uint64_t *dst, const uint64_t *src, uint32_t lm, u
     // 2. block DIT over the low L2 bits, then 3. strided DIT over n1
     uint32_t L2 = lm < NTT_LOG_TILE ? lm : NTT_LOG_TILE, L1 = lm - L2;
     if (L1 > 2 * NTT_MAX_STRIDED) return -2;
+    if (mx_split(lm, 0, &L1, &L2)) {
+        if (inverse) {
+            launch_block_mx<true, true>(dst, M, dst, M, L1, L2, 0, ncols, tb, st);
+            launch_strided_mx(strided_fwd_mx<true>, dst, M, L1, L2, ncols, tb, st);
+        } else {
+            launch_block_mx<true, false>(dst, M, dst, M, L1, L2, 0, ncols, tb, st);
+            launch_strided_mx(strided_fwd_mx<false>, dst, M, L1, L2, ncols, tb, st);
+        }
+        return (int)hipGetLastError();
+    }
     dim3 g(1u << L1, (unsigned)ncols);
     if (inverse)
         hipLaunchKernelGGL((L1 > NTT_MAX_STRIDED ? k_lde_block<true, true, true> : k_lde_block<true, true, false>), g,

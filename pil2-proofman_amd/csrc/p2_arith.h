@@ -137,6 +137,37 @@ __device__ __forceinline__ uint64_t hz_fold(hz a)
     return gl_pack(r0, r1);
 }
 
+// Two halves-form folds in step
+__device__ __forceinline__ void hz_fold2(const hz *a, uint64_t *out)
+{
+    uint64_t r[2], d[2], c[2], bb[2];
+    asm("v_mad_u64_u32 %0, %2, %4, -1, %6\n\t"
+        "v_mad_u64_u32 %1, %3, %5, -1, %7"
+        : "=&v"(r[0]), "=&v"(r[1]), "=&s"(d[0]), "=&s"(d[1])
+        : "v"((uint32_t)(a[0].hi >> 32)), "v"((uint32_t)(a[1].hi >> 32)), "v"(a[0].lo), "v"(a[1].lo));
+    uint32_t r0[2], r1[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        r0[k] = (uint32_t)r[k];
+        r1[k] = (uint32_t)(r[k] >> 32);
+    }
+    asm("v_add_co_u32_e64 %[r1a], %[ca], %[r1a], %[h0a]\n\t"
+        "v_add_co_u32_e64 %[r1b], %[cb], %[r1b], %[h0b]\n\t"
+        "s_nop 0\n\t"
+        "v_subb_co_u32_e64 %[r0a], %[ba], %[r0a], 0, %[ca]\n\t"
+        "v_subb_co_u32_e64 %[r0b], %[bb], %[r0b], 0, %[cb]\n\t"
+        "s_andn2_b64 %[ca], %[ca], %[ba]\n\t"
+        "s_andn2_b64 %[cb], %[cb], %[bb]\n\t"
+        "v_addc_co_u32_e64 %[r1a], %[ba], %[r1a], 0, %[ca]\n\t"
+        "v_addc_co_u32_e64 %[r1b], %[bb], %[r1b], 0, %[cb]"
+        : [r0a] "+v"(r0[0]), [r0b] "+v"(r0[1]), [r1a] "+v"(r1[0]), [r1b] "+v"(r1[1]), [ca] "=&s"(c[0]), [cb] "=&s"(c[1]),
+          [ba] "=&s"(bb[0]), [bb] "=&s"(bb[1])
+        : [h0a] "v"((uint32_t)a[0].hi), [h0b] "v"((uint32_t)a[1].hi)
+        : "scc");
+#pragma unroll
+    for (int k = 0; k < 2; k++) out[k] = gl_pack(r0[k], r1[k]);
+}
+
 // a*b mod p as a 64-bit word (any 64-bit a, b)
 __device__ __forceinline__ uint64_t p2_mul(uint64_t a, uint64_t b) { return gl_mulk1(a, b, 0, 0); }
 
@@ -179,6 +210,7 @@ __device__ void p2_mul3(const uint64_t *a, const uint64_t *b, uint64_t *out);
 __device__ void p2_mul_add3(const uint64_t *a, const uint64_t *b, uint32_t s_lo, uint32_t s_hi, uint64_t *out);
 __device__ void hz_fold3(const hz *a, uint64_t *out);
 __device__ uint64_t hz_fold(hz a);
+__device__ void hz_fold2(const hz *a, uint64_t *out);
 __device__ uint64_t lz_fold(lz a);
 __device__ uint64_t p2_mul(uint64_t a, uint64_t b);
 __device__ void p2_mul2(const uint64_t *a, const uint64_t *b, uint64_t *out);

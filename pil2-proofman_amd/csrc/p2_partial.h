@@ -19,11 +19,10 @@
 // lanes l and l + 32 and whole operands (111 -> 81 products a segment at width 12, leaves
 // of 2^20 x 128 rows 4.37 -> 4.10 ms).
 //
-// Bytes are signed in the instruction: words enter as w ^ 0x8080808080808080, i.e.
-// byte - 128, and 128 * (sum of the coefficients) * 0x0101010101010101 goes into the
-// result's constant together with the round constant that follows it.
+// (Bytes, digits and addends: gl_digits.h. The addend of a result carries the round
+// constant that is added to it next.)
 #pragma once
-#include "p2_arith.h"
+#include "gl_digits.h"
 #include "p2_constants.h"
 
 #define P2_SEG 11  // rounds per segment (odd: y_1 .. y_10 fill whole operands)
@@ -31,8 +30,9 @@
 
 namespace p2c {
 
-constexpr uint64_t add(uint64_t a, uint64_t b) { return a >= GL_P - b ? a - (GL_P - b) : a + b; }
-constexpr uint64_t mul(uint64_t a, uint64_t b) { return (uint64_t)((unsigned __int128)a * b % GL_P); }
+using glc::add;
+using glc::addends;
+using glc::mul;
 
 constexpr uint64_t rc8[86] = P2_RC8_INIT, rc12[118] = P2_RC12_INIT, rc16[150] = P2_RC16_INIT;
 constexpr uint64_t d8[8] = P2_DIAG8_INIT, d12[12] = P2_DIAG12_INIT, d16[16] = P2_DIAG16_INIT;
@@ -92,13 +92,8 @@ template <int W> struct Operands {
     {
         uint64_t v = c;
         for (int a = 0; a < 8; a++, v = mul(v, 256)) {
-            // v or v - p in the range of eight digits -128 .. 127; digit = byte or byte - 256
-            uint64_t x = v > 0x7F7F7F7F7F7F7F7FULL ? v - GL_P : v;
-            for (int t = 0; t < 8; t++) {
-                int64_t d = (int64_t)(int8_t)(x & 255);
-                b[at + t * 16 + a] = (int8_t)d;
-                x = (uint64_t)((int64_t)(x - (uint64_t)d) >> 8);
-            }
+            const glc::Digits d(v);
+            for (int t = 0; t < 8; t++) b[at + t * 16 + a] = d.d[t];
         }
     }
     constexpr void put(int n, int out0, int in0, bool half)
@@ -131,16 +126,6 @@ template <int W> struct Operands {
     }
 };
 
-// The constant v of a result as the two 64-bit addends of the halves form, with 2^47 in
-// each half, which makes the sums non-negative
-constexpr void addends(uint64_t v, uint64_t *k)
-{
-    const uint64_t bias = 1ULL << 47, off = add(bias, mul(bias, 1ULL << 32));
-    uint64_t d = add(v, GL_P - off);
-    k[0] = bias + (uint32_t)d;
-    k[1] = bias + (d >> 32);
-}
-
 // Per segment and out-word the addends of its result: the correction for the signed
 // bytes and the round constant added to the word next.
 template <int W> struct Addends {
@@ -152,7 +137,7 @@ template <int W> struct Addends {
             for (int o = 0; o < NOUT; o++) {
                 uint64_t s = 0;
                 for (int i = 0; i < Forms<W>::NIN; i++) s = add(s, forms<W>.c[o][i]);
-                uint64_t v = mul(mul(s, 128), 0x0101010101010101ULL % GL_P);
+                uint64_t v = mul(mul(s, 128), glc::kBytes);
                 int r = g * P2_SEG + o + 1;  // the partial round whose S-box takes out-word o (o = 10: w_0)
                 if (o < P2_SEG && r < P2_SEG * P2_SEGS) v = add(v, rc(W, 4 * W + r) % GL_P);
                 // after the last segment the first of the closing full rounds follows
@@ -179,8 +164,8 @@ template <int W> __constant__ const p2c::NextRc<W> c_p2_next_rc{};
 template <int W> __device__ const p2c::Operands<W> c_p2_operands{};
 template <int W> __constant__ const p2c::Addends<W> c_p2_addends{};
 
-typedef int p2_v4i __attribute__((ext_vector_type(4)));
-typedef int p2_v16i __attribute__((ext_vector_type(16)));
+typedef gl_v4i p2_v4i;
+typedef gl_v16i p2_v16i;
 
 #if defined(__HIP_DEVICE_COMPILE__)
 
@@ -227,13 +212,6 @@ __device__ __forceinline__ p2_rows p2_operand_rows(const p2_v4i *s)
     }
 P2_DIGITS(p2_digits, "s")
 P2_DIGITS(p2_digits_v, "v")
-
-// Bytes of a word as the signed bytes of half an operand
-__device__ __forceinline__ void p2_put_word(p2_v4i &v, int half, uint64_t w)
-{
-    v[2 * half] = (int)((uint32_t)w ^ 0x80808080u);
-    v[2 * half + 1] = (int)((uint32_t)(w >> 32) ^ 0x80808080u);
-}
 
 // The A operands on their way from LDS, P2_AHEAD of them (1 and 2 measure the same within
 // 2 %; more pushes width 16 further over 128 VGPRs). First those of the u, then the state's.
@@ -296,11 +274,11 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int 
     p2_stream<W> st;
     st.start(ops);
 #pragma unroll
-    for (int i = 1; i < W; i++) p2_put_word(in[(i - 1) / 2], (i - 1) % 2, s[i]);
+    for (int i = 1; i < W; i++) gl_put_word(in[(i - 1) / 2], (i - 1) % 2, s[i]);
     p2_v16i acc = {}, nxt;
 #pragma unroll
     for (int t = 0; t < NS - 1; t++) st.mac(acc, in[t]);
-    p2_put_word(in[NS - 1], 1, pow7(s[0]));
+    gl_put_word(in[NS - 1], 1, pow7(s[0]));
     st.mac(acc, in[NS - 1]);
 #pragma unroll
     for (int p = 0; p < NU; p++) {
@@ -309,14 +287,14 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int 
 #pragma unroll
         for (int t = 0; t < NS + p && p + 1 < NU; t++) st.mac(nxt, in[t]);
         uint64_t y = pow7(hz_fold(u));
-        p2_put_word(in[NS + p], 0, y);
-        p2_put_word(in[NS + p], 1, y);  // any value: its coefficients in the next operand are zero
+        gl_put_word(in[NS + p], 0, y);
+        gl_put_word(in[NS + p], 1, y);  // any value: its coefficients in the next operand are zero
         st.mac(acc, in[NS + p]);
         u = p2_digits(acc, 8, k[2 * p + 1], c16);
         // the first word's sums are written again by the second product: they stay
         // reserved until its results have been read
         asm volatile("" : "+v"(u.lo) : "v"(acc));
-        p2_put_word(in[NS + p], 1, pow7(hz_fold(u)));
+        gl_put_word(in[NS + p], 1, pow7(hz_fold(u)));
         if (p + 1 < NU) st.mac(nxt, in[NS + p]);
         acc = nxt;
     }

@@ -51,12 +51,8 @@ template <int W> struct RowOps {
     {
         uint64_t v = c;
         for (int a = 0; a < 8; a++, v = mul(v, 256)) {
-            uint64_t x = v > 0x7F7F7F7F7F7F7F7FULL ? v - GL_P : v;
-            for (int t = 0; t < 8; t++) {
-                int64_t d = (int64_t)(int8_t)(x & 255);
-                b[(t < 4 ? at0 : at1) + (kg * rows + row + t % 4) * 16 + slot * 8 + a] = (int8_t)d;
-                x = (uint64_t)((int64_t)(x - (uint64_t)d) >> 8);
-            }
+            const glc::Digits d(v);
+            for (int t = 0; t < 8; t++) b[(t < 4 ? at0 : at1) + (kg * rows + row + t % 4) * 16 + slot * 8 + a] = d.d[t];
         }
     }
     constexpr RowOps() : b{}
@@ -102,7 +98,7 @@ template <int W> struct RowAddends {
         for (int w = 0; w < W; w++) {
             int m = m4[w % 4][0] + m4[w % 4][1] + m4[w % 4][2] + m4[w % 4][3];
             for (int r = 0; r < 9; r++) {
-                uint64_t v = mul(128 * 5 * (uint64_t)m, 0x0101010101010101ULL % GL_P);
+                uint64_t v = mul(128 * 5 * (uint64_t)m, glc::kBytes);
                 v = add(v, (r == 0 ? rc(W, w) : next.k[r - 1][w]) % GL_P);
                 addends(v, ext[r][w]);
             }
@@ -126,38 +122,6 @@ template <int CTRL>
 __device__ __forceinline__ int p2_dpp(int v)
 {
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, false);
-}
-
-__device__ __forceinline__ void p2_mac16(p2_v4i &acc, const p2_v4i &a, const p2_v4i &in)
-{
-    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, in, acc, 0, 0, 0);
-}
-
-// The word whose digit sums are a (digits 0 .. 3) and b (4 .. 7), with addends k0, k1 of
-// the lane's own or (SK) in scalar registers
-template <bool SK>
-__device__ __forceinline__ uint64_t p2_word16(const p2_v4i &a, const p2_v4i &b, uint64_t k0, uint64_t k1)
-{
-    const uint32_t c16 = 65536;
-    uint32_t e0 = ((uint32_t)a[1] << 8) + (uint32_t)a[0], e1 = ((uint32_t)a[3] << 8) + (uint32_t)a[2];
-    uint32_t e2 = ((uint32_t)b[1] << 8) + (uint32_t)b[0], e3 = ((uint32_t)b[3] << 8) + (uint32_t)b[2];
-    uint64_t l, h, d0, d1;
-    if constexpr (SK)
-        asm("v_mad_i64_i32 %0, %2, %4, %6, %7\n\t"
-            "v_mad_i64_i32 %1, %3, %5, %6, %8"
-            : "=&v"(l), "=&v"(h), "=&s"(d0), "=&s"(d1)
-            : "v"(e1), "v"(e3), "v"(c16), "s"(k0), "s"(k1));
-    else
-        asm("v_mad_i64_i32 %0, %2, %4, %6, %7\n\t"
-            "v_mad_i64_i32 %1, %3, %5, %6, %8"
-            : "=&v"(l), "=&v"(h), "=&s"(d0), "=&s"(d1)
-            : "v"(e1), "v"(e3), "v"(c16), "v"(k0), "v"(k1));
-    hz r;
-    asm("v_mad_i64_i32 %0, %2, %4, 1, %6\n\t"
-        "v_mad_i64_i32 %1, %3, %5, 1, %7"
-        : "=&v"(r.lo), "=&v"(r.hi), "=&s"(d0), "=&s"(d1)
-        : "v"(e0), "v"(e2), "v"(l), "v"(h));
-    return hz_fold(r);
 }
 
 // What was loaded in program order before is requested before what follows from x
@@ -215,11 +179,11 @@ template <int W> struct p2_row {
         p2_v4i b0 = {lo, hi, p2_dpp<0xB1>(lo), p2_dpp<0xB1>(hi)};
         p2_v4i b1 = {p2_dpp<0x4E>(lo), p2_dpp<0x4E>(hi), p2_dpp<0x1B>(lo), p2_dpp<0x1B>(hi)};
         p2_v4i a = {}, b = {};
-        p2_mac16(a, ext[0], b0);
-        p2_mac16(b, ext[2], b0);
-        p2_mac16(a, ext[1], b1);
-        p2_mac16(b, ext[3], b1);
-        return p2_word16<false>(a, b, k0, k1);
+        gl_mac16(a, ext[0], b0);
+        gl_mac16(b, ext[2], b0);
+        gl_mac16(a, ext[1], b1);
+        gl_mac16(b, ext[3], b1);
+        return hz_fold(gl_digit_sums<false>(a, b, k0, k1));
     }
     // full rounds r .. r + 3: S-box, external layer, next constants
     __device__ __forceinline__ uint64_t full(uint64_t x, int r0) const
@@ -290,8 +254,8 @@ template <int W> struct p2_row {
 #pragma unroll
             for (int t = 0; t < NT; t++)
                 if (e + 1 < P2_SEG && t < Op::tiles(e) && t != tn) {
-                    p2_mac16(a, cur[0][t], in[t]);
-                    p2_mac16(b, cur[1][t], in[t]);
+                    gl_mac16(a, cur[0][t], in[t]);
+                    gl_mac16(b, cur[1][t], in[t]);
                 }
             if (e + 1 < P2_SEG) operands(nxt, e + 1);
             p2_loads_first(u);
@@ -299,9 +263,9 @@ template <int W> struct p2_row {
             in[tn][s % 2 * 2] = g == (uint32_t)gn ? (int)((uint32_t)y ^ 0x80808080u) : in[tn][s % 2 * 2];
             in[tn][s % 2 * 2 + 1] = g == (uint32_t)gn ? (int)((uint32_t)(y >> 32) ^ 0x80808080u) : in[tn][s % 2 * 2 + 1];
             if (e + 1 < P2_SEG) {
-                p2_mac16(a, cur[0][tn], in[tn]);
-                p2_mac16(b, cur[1][tn], in[tn]);
-                u = p2_word16<true>(a, b, k[e][0], k[e][1]);
+                gl_mac16(a, cur[0][tn], in[tn]);
+                gl_mac16(b, cur[1][tn], in[tn]);
+                u = hz_fold(gl_digit_sums<true>(a, b, k[e][0], k[e][1]));
 #pragma unroll
                 for (int t = 0; t < NT; t++) cur[0][t] = nxt[0][t], cur[1][t] = nxt[1][t];
             }
@@ -318,8 +282,8 @@ template <int W> struct p2_row {
             }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                p2_mac16(sa, cur[0][t], in[t]);
-                p2_mac16(sb, cur[1][t], in[t]);
+                gl_mac16(sa, cur[0][t], in[t]);
+                gl_mac16(sb, cur[1][t], in[t]);
             }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -327,7 +291,7 @@ template <int W> struct p2_row {
                 b[i] = w == 0 || q == (uint32_t)w ? sb[i] : b[i];
             }
         }
-        return p2_word16<false>(a, b, ks0, ks1);
+        return hz_fold(gl_digit_sums<false>(a, b, ks0, ks1));
     }
     // The permutation: word `word` in and out. need_stage (the same for the block, whose
     // threads then all call it): no stage() yet since start().

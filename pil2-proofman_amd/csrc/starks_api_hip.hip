@@ -186,9 +186,8 @@ static int64_t check_arity(uint64_t arity)
     return 0;
 }
 
-// measured on the plain workloads: 2^13 strided tiles (two blocks per CU) and radix-16
-// block rounds (plain-large 118.9 ms against 119.4 ms with radix-8 rounds, now that blowup
-// 4 runs two columns per block; plain-small the same either way)
+// Tile and radix matter only to the shapes whose transform rounds stay on the VALU
+// (blowups above 8, above 2^24 rows): 2^13 tiles, two blocks per CU, and radix-16 rounds
 static const Pil2CommitPlan kDefaultPlan = {1, 13, 4, P2_COOP_MAX_PARENTS};
 
 static int64_t lde_impl(uint64_t *d_lde, const uint64_t *d_trace, uint64_t *d_scratch, uint64_t nBits,

@@ -1,0 +1,76 @@
+"""GPU tests of the transforms' rounds on the matrix cores: every number of strided bits and
+short-round bits, every blowup, odd column counts, words at and past p, and the shapes next
+to those that keep the rounds on the VALU, against the oracle."""
+import numpy as np
+import pytest
+
+from golden_helpers import colmajor_to_rowmajor
+import datagen
+
+pytestmark = pytest.mark.gpu
+P = 0xFFFFFFFF00000001
+
+
+@pytest.fixture(scope="module")
+def pc():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("GPU test run without a HIP device")
+    import pil2_commit
+    pil2_commit.set_hash_family(2)
+    return pil2_commit
+
+
+def _words(n, seed):
+    """n words, some of them at and past p, and the same residues below p."""
+    raw = datagen.uniform(n, seed)
+    raw[::5] = np.array([0, 1, P - 1, P, P + 1, 2**64 - 1, 2**32 - 1], dtype=np.uint64)[np.arange(raw[::5].size) % 7]
+    return raw, np.where(raw >= np.uint64(P), raw - np.uint64(P), raw)
+
+
+LDE = [(10, 0, 2), (11, 0, 3), (12, 0, 1), (14, 0, 2), (15, 0, 1), (17, 0, 2), (18, 0, 3), (19, 0, 1),
+       (9, 1, 3), (10, 1, 2), (13, 1, 1), (14, 1, 3), (15, 1, 2), (16, 1, 5), (17, 1, 1), (18, 1, 2), (21, 1, 1),
+       (22, 1, 1), (8, 2, 2), (9, 2, 3), (12, 2, 2), (13, 2, 5), (14, 2, 1), (15, 2, 4), (17, 2, 3), (18, 2, 2),
+       (7, 3, 3), (8, 3, 2), (9, 3, 1), (11, 3, 5), (12, 3, 3), (13, 3, 2), (16, 3, 1), (17, 3, 3), (20, 3, 1),
+       (10, 4, 3), (13, 4, 2)]
+
+
+@pytest.mark.parametrize("nb,lb,cols", LDE)
+def test_lde(pc, oracle, nb, lb, cols):
+    import torch
+    n, ne = 1 << nb, 1 << (nb + lb)
+    raw, trace = _words(n * cols, 7000 + 40 * nb + lb)
+    out = pc.empty(ne * cols)
+    pc.NTT_Goldilocks(n).LDE(out, pc.to_device(raw.reshape(n, cols)), ne, n, cols)
+    torch.cuda.synchronize()
+    got = colmajor_to_rowmajor(pc.to_host(out), ne, cols)
+    assert (got == oracle.lde(trace.reshape(n, cols), ne)).all()
+
+
+@pytest.mark.parametrize("lg,cols", [(10, 2), (11, 3), (14, 1), (15, 2), (16, 3), (17, 1), (19, 2), (21, 1), (22, 1)])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_ntt(pc, oracle, lg, cols, inverse):
+    import torch
+    n = 1 << lg
+    raw, a = _words(n * cols, 8000 + lg)
+    d = pc.to_device(raw)
+    ntt = pc.NTT_Goldilocks(n)
+    (ntt.INTT if inverse else ntt.NTT)(None, d, n, cols, row_major=False)
+    torch.cuda.synchronize()
+    f = oracle.intt if inverse else oracle.ntt
+    got = pc.to_host(d).reshape(cols, n)
+    for c in range(cols):
+        assert (got[c] == f(a.reshape(cols, n)[c])).all()
+
+
+@pytest.mark.parametrize("nb,lb,qdeg,qdim", [(11, 0, 1, 3), (13, 1, 2, 3), (16, 1, 2, 1), (17, 1, 1, 3), (12, 2, 4, 3),
+                                             (14, 2, 3, 3), (18, 2, 4, 1), (8, 3, 8, 3), (12, 3, 5, 3), (16, 3, 8, 1),
+                                             (9, 4, 3, 3)])
+def test_compute_q(pc, oracle, nb, lb, qdeg, qdim):
+    import torch
+    ne = 1 << (nb + lb)
+    raw, q = _words(ne * qdim, 9000 + 40 * nb + lb)
+    cm, _ = pc.compute_q(pc.to_device(raw), nb, nb + lb, qdeg, q_dim=qdim, arity=3, row_major=True)
+    torch.cuda.synchronize()
+    got = colmajor_to_rowmajor(pc.to_host(cm), ne, qdeg * qdim)
+    assert (got == oracle.compute_q(q.reshape(ne, qdim), 1 << nb, qdeg)).all()
