@@ -544,18 +544,19 @@ int64_t pil2hip_ntt(uint64_t *d_dst, const uint64_t *d_src, uint64_t *d_scratch,
         NttTablesHost *tb;
         int64_t rc = ensure_tables(&tb);
         if (rc) return rc;
-        if (rowMajor) {  // rows -> columns, transform out of place, columns -> rows
+        if (rowMajor) {  // rows -> bit-reversed columns, transform, columns -> rows
             if (!d_scratch) return fail(-13, "row-major transforms need a scratch of 2 * 2^nBits * nCols words");
             uint64_t *a = d_scratch, *b = d_scratch + M * nCols;
-            e = ntt_launch_rm2cm(a, d_src, M, nCols, nCols, M, st);
-            if (!e) e = ntt_launch_ntt(b, a, (uint32_t)nBits, nCols, inverse, tb, st);
-            if (!e) e = ntt_launch_cm2rm(d_dst, b, M, nCols, M, nCols, st);
+            e = ntt_launch_bitrev_rows(a, b, d_src, (uint32_t)nBits, nCols, inverse, st);
+            if (!e) e = ntt_launch_reversed(a, a, (uint32_t)nBits, nCols, inverse, tb, st);
+            if (!e) e = ntt_launch_cm2rm(d_dst, a, M, nCols, M, nCols, st);
         } else if (d_dst == d_src) {
             if (!d_scratch) return fail(-13, "in-place column-major transforms need a scratch of 2^nBits * nCols words");
-            e = ntt_launch_ntt(d_scratch, d_src, (uint32_t)nBits, nCols, inverse, tb, st);
-            if (!e) e = (int)hipMemcpyAsync(d_dst, d_scratch, M * nCols * 8, hipMemcpyDeviceToDevice, st);
+            e = ntt_launch_bitrev(d_scratch, d_src, (uint32_t)nBits, nCols, inverse, st);
+            if (!e) e = ntt_launch_reversed(d_dst, d_scratch, (uint32_t)nBits, nCols, inverse, tb, st);
         } else {
-            e = ntt_launch_ntt(d_dst, d_src, (uint32_t)nBits, nCols, inverse, tb, st);
+            e = ntt_launch_bitrev(d_dst, d_src, (uint32_t)nBits, nCols, inverse, st);
+            if (!e) e = ntt_launch_reversed(d_dst, d_dst, (uint32_t)nBits, nCols, inverse, tb, st);
         }
     }
     if (e < 0) return fail(-14, "NTT plan not supported for this shape");

@@ -74,3 +74,41 @@ def test_compute_q(pc, oracle, nb, lb, qdeg, qdim):
     torch.cuda.synchronize()
     got = colmajor_to_rowmajor(pc.to_host(cm), ne, qdeg * qdim)
     assert (got == oracle.compute_q(q.reshape(ne, qdim), 1 << nb, qdeg)).all()
+
+
+@pytest.mark.parametrize("lg,cols", [(4, 8), (5, 1), (6, 9), (11, 8), (12, 7), (12, 64), (13, 65), (15, 50)])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_ntt_rows(pc, oracle, lg, cols, inverse):
+    """Row-major transforms: about the width of the tile that transposes and reverses, fewer
+    rows than it has, one column and many; in place and not."""
+    import torch
+    n = 1 << lg
+    raw, a = _words(n * cols, 8500 + lg * 70 + cols)
+    ntt = pc.NTT_Goldilocks(n)
+    run = ntt.INTT if inverse else ntt.NTT
+    src = pc.to_device(raw)
+    dst = pc.empty(n * cols)
+    run(dst, src, n, cols, row_major=True)
+    torch.cuda.synchronize()
+    assert (pc.to_host(src) == raw).all()
+    run(None, src, n, cols, row_major=True)
+    torch.cuda.synchronize()
+    f = oracle.intt if inverse else oracle.ntt
+    want = np.stack([f(a.reshape(n, cols)[:, c]) for c in range(cols)], axis=1)
+    assert (pc.to_host(dst).reshape(n, cols) == want).all()
+    assert (pc.to_host(src).reshape(n, cols) == want).all()
+
+
+@pytest.mark.parametrize("lg,cols", [(22, 4), (22, 5)])
+def test_ntt_rows_long(pc, lg, cols):
+    """The longest narrow rows that go through one pass, and longer: as the columns do."""
+    import torch
+    n = 1 << lg
+    raw, _ = _words(n * cols, 8900 + cols)
+    ntt = pc.NTT_Goldilocks(n)
+    rows = pc.to_device(raw)
+    columns = rows.reshape(n, cols).t().contiguous().reshape(-1)
+    ntt.INTT(None, rows, n, cols, row_major=True)
+    ntt.INTT(None, columns, n, cols, row_major=False)
+    torch.cuda.synchronize()
+    assert torch.equal(rows.reshape(n, cols), columns.reshape(cols, n).t())
