@@ -19,6 +19,7 @@ struct NttSplitTables {
 
 struct NttTablesHost {
     uint64_t *tkf, *tki;                   // 2^15 entries each: [2^k + y] = w_{2^k}^(+-y), k <= 14
+    uint64_t *dtf, *dti;                   // 2^15 entries each: the same by a round's values
     NttSplitTables split[2];               // [0]: the 2^24 domain (bits 12), [1]: 2^28 (bits 14)
 };
 

@@ -37,12 +37,14 @@
 //   tkf[2^k + y] = w_{2^k}^y, tki[2^k + y] = w_{2^k}^-y  (k <= 14, y < 2^k)  inside tiles:
 //        one compact table per round size, so a round's twiddles of 2^k <= 2^12
 //        entries fit the 32 KiB L1 instead of being spread over a 2^14-entry table
+//   dtf[2^k + (i << (k - 4)) + o] = w_{2^k}^(o bitrev4(i)), dti with w^-1 (4 <= k <= 14):
+//        a round's twiddles on the matrix cores, in the order of the round's values
 //   twl/twh: w_D^x = lo[x & (2^bits - 1)] * hi[x >> bits]   (x < D)   between passes
 //   shl/shh: 7^e = lo[e & (2^bits - 1)] * hi[e >> bits]              coset shift
 // over the domain D = 2^(2*bits): bits = 12 (D = 2^24, lo tables of 32 KiB) for
 // transforms up to 2^24 points, bits = 14 (D = 2^28) above that.
 struct NttTables {
-    const uint64_t *tkf, *tki;
+    const uint64_t *tkf, *tki, *dtf, *dti;
     const uint64_t *twl_f, *twh_f, *twl_i, *twh_i;
     const uint64_t *shl, *shh;
     uint32_t bits;
@@ -52,7 +54,7 @@ struct NttTables {
 static NttTables tables_for(const NttTablesHost *th, uint32_t log_max)
 {
     const NttSplitTables &S = th->split[log_max > 24 ? 1 : 0];
-    return {th->tkf, th->tki, S.twl_f, S.twh_f, S.twl_i, S.twh_i, S.shl, S.shh, S.bits};
+    return {th->tkf, th->tki, th->dtf, th->dti, S.twl_f, S.twh_f, S.twl_i, S.twh_i, S.shl, S.shh, S.bits};
 }
 
 __device__ __forceinline__ uint32_t tw_lo(uint32_t x, const NttTables &tb) { return x & ((1u << tb.bits) - 1u); }

@@ -82,7 +82,7 @@ template <int KIND, int R, int S> __device__ const nttc::Mat<KIND, R, S> c_ntt_m
 // step, gi < step: their indices have no bits in common, so an address is a lane's part
 // for gi plus a scalar part for c.
 struct MxLane {
-    uint32_t g, gi, first, step, br;  // first: the wave's gi (scalar), br: the two bits of g exchanged
+    uint32_t g, gi, first, step;  // first: the wave's gi (scalar)
 };
 
 // Shapes of the strided passes and of the block pass (below)
@@ -109,7 +109,7 @@ __device__ __forceinline__ MxLane mx_lane()
 {
     const uint32_t l = mx_lane_id(), g = l >> 4;
     uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    return {g, wave * 16 + (l & 15), wave * 16, (blockDim.x >> 6) * 16, (g & 1) * 2 + (g >> 1)};
+    return {g, wave * 16 + (l & 15), wave * 16, (blockDim.x >> 6) * 16};
 }
 
 // The group's bits gi of a round over index bits [q, q + 4) of a tile with 2^lt lines: the
@@ -196,10 +196,22 @@ __device__ __forceinline__ void mx_canon4(uint64_t *v)
     gl_canon2(v + 2);
 }
 
-// w[i] = w^(o * bitrev4(g + 4i)) for the root w of the table t of 2^lg powers
-__device__ __forceinline__ void mx_twiddles(uint64_t *w, const uint64_t *t, uint32_t o, const MxLane &L)
+// w[i] = w^(o * bitrev4(g + 4i)), o < 2^q, w of order 2^(q + 4): the round table t has them
+// at the values' places, so that a wave reads runs (by exponent, 16 lanes with consecutive
+// o read up to 16 lines, and of a table larger than the L1 cache one word of each: block
+// pass of 2^22 x 128 to 2^24 16.0 ms instead of 15.4, INTT of 2^21 x 24 405 us instead of 385)
+__device__ __forceinline__ void mx_twiddles(uint64_t *w, const uint64_t *t, uint32_t o, uint32_t q, const MxLane &L)
 {
-    const uint32_t o8 = o * 8, b = __umul24(o8, 4 * L.br);
+    const uint32_t off = 8 * ((L.g << q) | o);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) w[i] = mx_ld(t + ((4 * i) << q), off);
+}
+
+// The same by exponent, from the powers t of w: for the strided passes, whose lanes have few
+// different o and whose tables the L1 cache holds; it takes fewer registers
+__device__ __forceinline__ void mx_powers(uint64_t *w, const uint64_t *t, uint32_t o, const MxLane &L)
+{
+    const uint32_t o8 = o * 8, b = __umul24(o8, 4 * ((L.g & 1) * 2 + (L.g >> 1)));
     w[0] = mx_ld(t, b);
     w[1] = mx_ld(t, b + 2 * o8);
     w[2] = mx_ld(t, b + o8);
@@ -239,9 +251,9 @@ struct MxTile {
     }
 };
 
-// A full round in LDS (twiddles from the table t of 2^(q + 4) powers): DIT twiddles before
+// A full round in LDS (t: its table of 2^(q + 4) words, by place or by exponent): DIT twiddles before
 // the transform, DIF after it.
-template <int PIECES, int KIND, int S>
+template <int PIECES, bool PLACE = true, int KIND, int S>
 __device__ __forceinline__ void mx_round(uint64_t *__restrict__ s, const MxDft<KIND, 4, S> &d, uint32_t q, uint32_t lt,
                                          const uint64_t *t)
 {
@@ -252,7 +264,10 @@ __device__ __forceinline__ void mx_round(uint64_t *__restrict__ s, const MxDft<K
         uint64_t v[4], w[4];
         const uint32_t a = T.piece(c, L);
         T.read(v, s, a);
-        mx_twiddles(w, t, T.low(c, L), L);
+        if (PLACE)
+            mx_twiddles(w, t, T.low(c, L), q, L);
+        else
+            mx_powers(w, t, T.low(c, L), L);
         if (KIND != nttc::DIF_INV) mx_mul4(v, w);
         d.apply(v);
         if (KIND == nttc::DIF_INV) mx_mul4(v, w);
@@ -344,7 +359,7 @@ __global__ __launch_bounds__(512, 4) void k_ntt_strided_inv_mx(uint64_t *__restr
                 uint64_t w[4], *x = v[c & 1];
                 d.apply(x);
                 mx_fence();
-                mx_twiddles(w, tb.tki + (1u << L1), F.low(c, L), L);
+                mx_powers(w, tb.tki + (1u << L1), F.low(c, L), L);
                 mx_mul4(x, w);
                 F.write(s, F.piece(c, L), x);
                 mx_fence();
@@ -352,7 +367,7 @@ __global__ __launch_bounds__(512, 4) void k_ntt_strided_inv_mx(uint64_t *__restr
             }
             mx_sync();
             if constexpr (NR == 3) {
-                mx_round<MX_PIECES>(s, d, top - 4, lt, tb.tki + (1u << top));
+                mx_round<MX_PIECES, false>(s, d, top - 4, lt, tb.tki + (1u << top));
                 mx_sync();
             }
         }
@@ -407,7 +422,7 @@ __global__ __launch_bounds__(512, 4) void k_ntt_strided_fwd_mx(uint64_t *__restr
     constexpr int KIND = INV ? nttc::DIT_INV : nttc::DIT, NR = (L1 + 3) / 4, R = L1 - 4 * (NR - 1);
     constexpr uint32_t q = L1 - 4;
     const uint32_t lt = p.lt;
-    const uint64_t *tk = INV ? tb.tki : tb.tkf;
+    const uint64_t *tk = INV ? tb.dti : tb.dtf;
     MxDft<KIND, 4> d;
     if (R == 4) d.load();
     uint32_t tile = blockIdx.x;
@@ -475,7 +490,7 @@ __global__ __launch_bounds__(512, 4) void k_ntt_strided_fwd_mx(uint64_t *__restr
             for (uint32_t c = 0; c < MX_PIECES; c++) {
                 uint64_t v[4], w[4];
                 T.read(v, s, T.piece(c, L));
-                mx_twiddles(w, tk + (1u << L1), T.low(c, L), L);
+                mx_twiddles(w, tk + (1u << L1), T.low(c, L), q, L);
                 mx_mul4(v, w);
                 d.apply(v);
                 mx_canon4(v);
@@ -500,7 +515,7 @@ __global__ __launch_bounds__(512, 4) void k_ntt_strided_fwd_mx(uint64_t *__restr
 // The last round of phase 1 (2^R points, no twiddles), scaled by 7^e, e = bitrev(m 2^L2 +
 // k); kept in `held`, or (IN_PLACE) written back. A lane's four k differ in the same two
 // bits in every piece, so it takes one power a piece and the ratios once.
-template <int R, int TP, bool IN_PLACE>
+template <int R, int TP, bool IN_PLACE, bool PARTIAL>
 __device__ __forceinline__ void mx_block_coef(uint64_t *__restrict__ s, const MxDft<nttc::DIF_INV, R> &d,
                                               uint64_t (&held)[TP][4], uint32_t m, uint32_t L2, uint32_t log_n,
                                               uint32_t end, const NttTables &tb)
@@ -514,7 +529,7 @@ __device__ __forceinline__ void mx_block_coef(uint64_t *__restrict__ s, const Mx
     for (uint32_t i = 1; i < 4; i++) ratio[i] = mx_split_root(tb.shl, tb.shh, bitrev32(4 * i, log_n), tb);
 #pragma unroll
     for (uint32_t c = 0; c < TP; c++) {
-        if (L.first + c * L.step >= end) break;
+        if (PARTIAL && L.first + c * L.step >= end) break;
         uint64_t v[4], w[4];
         w[0] = mx_split_root(tb.shl, tb.shh, e0 + bitrev32(mx_pos(c * L.step, 0, 0) & mask, log_n), tb);
         T.read(v, s, T.piece(c, L));
@@ -558,6 +573,51 @@ __device__ __forceinline__ void mx_block_spread(uint64_t *__restrict__ s, const 
     }
 }
 
+// The same for R <= 2 on the VALU: a lane has groups of all 2^R values, and the block reads
+// one matrix less (2^18 x 75 to 2^20: block pass 537 -> 511 us). COEF_IN: they are read from
+// global memory (each copy reads them), not from where copy 0 stands, which saves a barrier;
+// with a matrix that would be reads of 32 bytes (2^15 x 50 NTT: 21.8 us instead of 17.7).
+template <bool INV, int R, int LOGB, bool COEF_IN>
+__device__ __forceinline__ void mx_block_spread_short(uint64_t *__restrict__ s, const uint64_t *__restrict__ src,
+                                                      const NttTables &tb)
+{
+    constexpr uint32_t N = 1 << R;
+    const uint32_t t = mx_thread(), o = t & ((1u << LOGB) - 1), grp = t >> LOGB;
+    const uint32_t at = 8 * lds_addr(grp << (R + LOGB)), copy = 8 * lds_addr(o);
+    uint64_t w[N];
+    if (LOGB > 0) {
+        const uint64_t *tk = (INV ? tb.tki : tb.tkf) + (1u << (LOGB + R));
+#pragma unroll
+        for (uint32_t i = 1; i < N; i++) w[i] = tk[o * bitrev32(i, R)];
+    }
+    uint64_t v[16 / N][N];
+#pragma unroll
+    for (uint32_t j = 0; j < 16 / N; j++) {
+        const uint32_t gj = (j * blockDim.x) >> LOGB;
+#pragma unroll
+        for (uint32_t i = 0; i < N; i++)
+            v[j][i] = COEF_IN ? mx_ld(src + (gj << R) + i, (grp << R) * 8)
+                              : mx_ld(s, at + 8 * (lds_addr(gj << (R + LOGB)) + lds_addr(i << LOGB)));
+    }
+    mx_fence();
+#pragma unroll
+    for (uint32_t j = 0; j < 16 / N; j++) {
+        const uint32_t gj = (j * blockDim.x) >> LOGB;
+        if (LOGB > 0) {
+            v[j][0] = gl_canon(v[j][0]);
+            gl_mul_v<N - 1>(v[j] + 1, v[j] + 1, w + 1);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < N; i += 2) gl_canon2(v[j] + i);
+        }
+        dft_dit<N, INV>(v[j]);
+#pragma unroll
+        for (uint32_t i = 0; i < N; i++)
+            mx_st(s, at + copy + 8 * (lds_addr(gj << (R + LOGB)) + lds_addr(i << LOGB)), v[j][i]);
+        mx_fence();
+    }
+}
+
 template <bool COEF_IN, bool INV, int LOGB, int R>
 __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
                                                           MxBlock p, NttTables tb)
@@ -575,7 +635,7 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
     const uint32_t lines = LINES == 2 && p.per == 2 && c0 + 1 < p.ncols ? 2 : 1;  // an odd last column is alone
     const uint64_t *src = in + c0 * p.cs_in + ((uint64_t)m << L2);
     uint64_t held[TP][4];
-    if constexpr (COEF_IN) {
+    if constexpr (COEF_IN && R >= 3) {
         constexpr uint32_t N = (1u << MX_LOG_THREAD) >> LOGB;
         uint64_t x[N];
 #pragma unroll
@@ -583,9 +643,9 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
 #pragma unroll
         for (uint32_t i = 0; i < N; i++) s[lds_addr((threadIdx.x + i * blockDim.x) << LOGB)] = x[i];
         mx_sync();
-    } else {
+    } else if constexpr (!COEF_IN) {
         const uint32_t q = L2 - 4, end = lines * per_line;
-        const bool busy = first < end;
+        const bool busy = LOGB < 2 || first < end;  // (without pairs every piece has a line)
         const MxLane L = mx_lane();
         const MxTile T(q, 0, L);  // (the line is the group's bits above the round's)
         MxDft<nttc::DIF_INV, 4> D;
@@ -595,23 +655,26 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
             // a wave's 16 groups are of one line
             const uint32_t off = ((L.g << q) | mx_low(L.gi, q, 0)) * 8;
             const uint64_t *line = src + (first >> q) * p.cs_in;
-#pragma unroll
-            for (uint32_t c = 0; c < TP; c++) {
-                if (first + c * step >= end) break;
+            auto load = [&](uint32_t c) {
+                if (LOGB >= 2 && first + c * step >= end) return;
                 const uint64_t *b = line + ((c * L.step) >> q) * p.cs_in + mx_low(c * L.step, q, 0);
 #pragma unroll
                 for (uint32_t i = 0; i < 4; i++) held[c][i] = mx_ld_nt(b + ((4 * i) << q), off);
-            }
+                mx_fence();
+            };
+            load(0);
+            if (TP > 1) load(1);
 #pragma unroll
             for (uint32_t c = 0; c < TP; c++) {
-                if (first + c * step >= end) break;
+                if (LOGB >= 2 && first + c * step >= end) break;
                 uint64_t w[4];
                 D.apply(held[c]);
                 mx_fence();
-                mx_twiddles(w, tb.tki + (1u << L2), T.low(c, L), L);
+                mx_twiddles(w, tb.dti + (1u << L2), T.low(c, L), q, L);
                 mx_mul4(held[c], w);
                 T.write(s, T.piece(c, L), held[c]);
                 mx_fence();
+                if (c + 2 < TP) load(c + 2);
             }
         }
         mx_sync();
@@ -619,9 +682,9 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
             qk -= 4;
             if (busy) {
                 if (LINES == 1 || TP == 1 || first + (TP - 1) * step < end)
-                    mx_round<TP>(s, D, qk, 0, tb.tki + (1u << (qk + 4)));
+                    mx_round<TP>(s, D, qk, 0, tb.dti + (1u << (qk + 4)));
                 else
-                    mx_round<(TP + 1) / 2>(s, D, qk, 0, tb.tki + (1u << (qk + 4)));
+                    mx_round<(TP + 1) / 2>(s, D, qk, 0, tb.dti + (1u << (qk + 4)));
             }
             mx_sync();
         }
@@ -631,13 +694,13 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
                 e = D;
             else
                 e.load();
-            mx_block_coef<R, TP, LOGB == 0>(s, e, held, m, L2, log_n, end, tb);
+            mx_block_coef<R, TP, LOGB == 0, (LOGB >= 2)>(s, e, held, m, L2, log_n, end, tb);
         }
         mx_sync();
     }
     const uint32_t e1 = bitrev32(m, L1), shift_e = 2 * tb.bits - (log_n + LOGB);
     const uint64_t *tl = INV ? tb.twl_i : tb.twl_f, *th = INV ? tb.twh_i : tb.twh_f;
-    const uint64_t *tk = INV ? tb.tki : tb.tkf;
+    const uint64_t *tk = INV ? tb.dti : tb.dtf;
 #pragma unroll 1
     for (uint32_t l = 0; l < lines; l++) {
         if constexpr (!COEF_IN && LOGB > 0) {
@@ -663,14 +726,17 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
             mx_sync();
         }
         MxDft<KIND, 4> F;
-        {
+        if constexpr (R <= 2) {
+            mx_block_spread_short<INV, R, LOGB, COEF_IN>(s, src, tb);
+            F.load();
+        } else if constexpr (R == 3) {
             MxDft<KIND, R> e;
             e.load();
             mx_block_spread<KIND, R, LOGB>(s, e, tb);
-            if constexpr (R == 4)
-                F = e;
-            else
-                F.load();
+            F.load();
+        } else {
+            F.load();
+            mx_block_spread<KIND, R, LOGB>(s, F, tb);
         }
         mx_sync();
         uint32_t q = LOGB + R;
@@ -701,7 +767,7 @@ __global__ __launch_bounds__(1024, 4) void k_lde_block_mx(const uint64_t *__rest
         for (uint32_t c = 0; c < MX_PIECES; c++) {
             uint64_t v[4], w[4];
             T.read(v, s, T.piece(c, L));
-            mx_twiddles(w, tk + (1u << top), T.low(c, L), L);
+            mx_twiddles(w, tk + (1u << top), T.low(c, L), q, L);
             mx_mul4(v, w);
             F.apply(v);
             if (L1) {  // the strided pass takes any words

@@ -62,7 +62,7 @@ static const int kMaxDevices = 16;
 // compact in-tile tables (2 x 2^15 words), then the split tables of the 2^24 domain
 // (6 x 2^12 words) and of the 2^28 domain (6 x 2^14 words)
 static const size_t kTabRoots = (size_t)2 << NTT_LOG_TILE, kTab24 = (size_t)1 << 12, kTab28 = (size_t)1 << 14;
-static const size_t kTabWords = 2 * kTabRoots + 6 * kTab24 + 6 * kTab28;
+static const size_t kTabWords = 4 * kTabRoots + 6 * kTab24 + 6 * kTab28;
 static __device__ __align__(256) uint64_t g_tab_dev[kTabWords];
 static NttTablesHost g_tables[kMaxDevices];
 static bool g_tables_ready[kMaxDevices];
@@ -94,7 +94,7 @@ static int64_t ensure_tables(NttTablesHost **out)
     if (!g_tables_ready[dev]) {
         const size_t nr = kTabRoots;
         std::vector<uint64_t> h(kTabWords);
-        uint64_t *rf = h.data(), *ri = rf + nr, *t24 = ri + nr, *t28 = t24 + 6 * kTab24;
+        uint64_t *rf = h.data(), *ri = rf + nr, *df = ri + nr, *di = df + nr, *t24 = di + nr, *t28 = t24 + 6 * kTab24;
         for (uint32_t k = 0; k <= NTT_LOG_TILE; k++) {  // rf[2^k + y] = w_{2^k}^y, ri[2^k + y] = w_{2^k}^-y
             uint64_t w = kRoots[k], wi = gl_inv(w), a = 1, b = 1;
             for (size_t y = 0; y < ((size_t)1 << k); y++) {
@@ -105,6 +105,14 @@ static int64_t ensure_tables(NttTablesHost **out)
             }
         }
         rf[0] = ri[0] = 1;  // unused slot
+        for (uint32_t k = 4; k <= NTT_LOG_TILE; k++) {  // df[2^k + (i << (k - 4)) + o] = w_{2^k}^(o bitrev4(i))
+            const size_t at = (size_t)1 << k;
+            for (size_t x = 0; x < at; x++) {
+                const size_t o = x & ((at >> 4) - 1), y = o * bitrev32((uint32_t)(x >> (k - 4)), 4);
+                df[at + x] = rf[at + y];
+                di[at + x] = ri[at + y];
+            }
+        }
         int ie = ntt_init_device();
         if (ie) return fail(-100 - ie, "NTT device init failed");
         split_tables(t24, 12);
@@ -115,9 +123,11 @@ static int64_t ensure_tables(NttTablesHost **out)
         NttTablesHost &T = g_tables[dev];
         T.tkf = dptr;
         T.tki = dptr + nr;
+        T.dtf = dptr + 2 * nr;
+        T.dti = dptr + 3 * nr;
         for (int d = 0; d < 2; d++) {
             size_t nt = d ? kTab28 : kTab24;
-            uint64_t *dt = dptr + 2 * nr + (d ? 6 * kTab24 : 0);
+            uint64_t *dt = dptr + 4 * nr + (d ? 6 * kTab24 : 0);
             NttSplitTables &S = T.split[d];
             S.twl_f = dt; S.twh_f = dt + nt; S.twl_i = dt + 2 * nt; S.twh_i = dt + 3 * nt; S.shl = dt + 4 * nt;
             S.shh = dt + 5 * nt;
