@@ -1114,8 +1114,10 @@ static bool mx_split(uint32_t log_n, uint32_t log_b, uint32_t *L1, uint32_t *L2)
 // instead of 4.12, but 2^16 x 100 to 2^18 365 us instead of 347, and 2^13 x 8 62 instead of 29.
 #define MX_PAIRS 8192
 // Strided tiles: four blocks of 256 threads a CU (2^18 x 75 forward 272 us; 292 with two of
-// 512 and 293 with eight of 128) while that leaves runs of whole 128-byte lines
-#define MX_STRIDED_TILE(L1) ((L1) <= 8 ? 12 : 13)
+// 512 and 293 with eight of 128), more where runs would be shorter than 128-byte lines
+// (2^22 x 128 to 2^24, 2^10 points: 11.05 ms forward and 3.2 ms inverse with one block of 1,024
+// threads a CU; 11.7 and 3.4 with two of 512, whose runs are half lines)
+#define MX_STRIDED_TILE(L1) ((L1) <= 8 ? 12 : (L1) + 4)
 #define MX_STRIDED_BLOCKS 1024  // of the launches that go on to further tiles
 
 static void launch_strided_mx(MxStridedKernel (*kernel)(uint32_t), uint64_t *data, uint64_t cs, uint32_t L1,

@@ -13,8 +13,8 @@
 // pass are the short ones; they are the rounds without twiddles.
 //
 // What bounds the passes (2^22 x 128 columns to 2^24, kernel times before, with the rounds
-// on the VALU, and now): block pass 19.3 -> 15.4 ms, strided forward 13.1 -> 11.7 ms,
-// strided inverse 3.8 -> 3.4 ms; at 75 columns 2^18 -> 2^20 the forward pass moves 4.4 TB/s of
+// on the VALU, and now): block pass 19.3 -> 15.4 ms, strided forward 13.1 -> 11.0 ms,
+// strided inverse 3.8 -> 3.2 ms; at 75 columns 2^18 -> 2^20 the forward pass moves 4.4 TB/s of
 // the 4.8 that a large copy reaches. VALU instructions fell by 40 percent, the matrix cores
 // are 20 percent busy; waiting (LDS, twiddles, barriers) is what is left, so registers are
 // held to 128 for four waves a SIMD: with 256 and two waves the same rounds took 16.8,
@@ -284,9 +284,7 @@ __device__ __forceinline__ void mx_round(uint64_t *__restrict__ s, const MxDft<K
 // block keeps its matrix and works on every gridDim.x-th tile of all columns.
 __device__ __forceinline__ uint64_t *mx_tile(uint64_t *data, const MxStrided &p, uint32_t tile)
 {
-    uint32_t bx = tile & ((1u << p.tiles_log) - 1);
-    // pairs that share 128-byte lines on blocks b and b + 8, as strided_tile
-    if (p.lt == 3 && p.tiles_log >= 4) bx = (bx & ~15u) | ((bx & 7u) << 1) | ((bx >> 3) & 1u);
+    const uint32_t bx = tile & ((1u << p.tiles_log) - 1);
     return data + (uint64_t)(tile >> p.tiles_log) * p.cs + ((uint64_t)bx << p.lt);
 }
 
@@ -325,7 +323,7 @@ __device__ __forceinline__ uint64_t mx_split_root(const uint64_t *tl, const uint
 // reads of 32 KB tables). Two reads for every word: 4.1 ms for 2^22 x 128 instead of 3.4. (L1 = 4:
 // m stays the same and the lines grow by a constant, and so the roots by a factor.)
 template <int L1>
-__global__ __launch_bounds__(512, 4) void k_ntt_strided_inv_mx(uint64_t *__restrict__ data, MxStrided p, NttTables tb)
+__global__ __launch_bounds__(1024, 4) void k_ntt_strided_inv_mx(uint64_t *__restrict__ data, MxStrided p, NttTables tb)
 {
     extern __shared__ uint64_t s[];
     constexpr int NR = (L1 + 3) / 4, R = L1 - 4 * (NR - 1);
@@ -416,7 +414,7 @@ __global__ __launch_bounds__(512, 4) void k_ntt_strided_inv_mx(uint64_t *__restr
 
 // NTT pass 3. The short round is the first one; the result is canonical.
 template <bool INV, int L1>
-__global__ __launch_bounds__(512, 4) void k_ntt_strided_fwd_mx(uint64_t *__restrict__ data, MxStrided p, NttTables tb)
+__global__ __launch_bounds__(1024, 4) void k_ntt_strided_fwd_mx(uint64_t *__restrict__ data, MxStrided p, NttTables tb)
 {
     extern __shared__ uint64_t s[];
     constexpr int KIND = INV ? nttc::DIT_INV : nttc::DIT, NR = (L1 + 3) / 4, R = L1 - 4 * (NR - 1);
