@@ -127,23 +127,21 @@ __device__ __forceinline__ void gl_prod_reduce3(const gl_prod *x, uint64_t *out)
 // Single product reduction (hazard gaps filled with s_nop).
 __device__ __forceinline__ uint64_t gl_prod_reduce1(gl_prod x)
 {
-    uint64_t r, c, b, m;
-    asm("v_mad_u64_u32 %0, %1, %2, -1, %3" : "=&v"(r), "=&s"(c) : "v"(x.x2), "v"(x.lo));
-    uint32_t r0 = (uint32_t)r, r1 = (uint32_t)(r >> 32), t0, t1;
+    uint64_t r = x.lo, c, b, m;
+    asm("v_mad_u64_u32 %0, %1, %2, -1, %0" : "+v"(r), "=s"(c) : "v"(x.x2));
+    uint32_t r0 = (uint32_t)r, r1 = (uint32_t)(r >> 32), x3 = x.x3;
     asm("v_sub_co_u32_e64 %[r0], %[b], %[r0], %[x3]\n\t"
         "s_nop 1\n\t"
         "v_subb_co_u32_e64 %[r1], %[b], %[r1], 0, %[b]\n\t"
-        "s_nop 1\n\t"
         "s_andn2_b64 %[m], %[c], %[b]\n\t"
         "s_andn2_b64 %[b], %[b], %[c]\n\t"
-        "v_cndmask_b32_e64 %[t0], 0, -1, %[m]\n\t"
-        "v_cndmask_b32_e64 %[t1], 0, -1, %[b]\n\t"
-        "v_cndmask_b32_e64 %[t0], %[t0], 1, %[b]\n\t"
-        "v_add_co_u32_e64 %[r0], %[c], %[r0], %[t0]\n\t"
-        "s_nop 1\n\t"
-        "v_addc_co_u32_e64 %[r1], %[c], %[r1], %[t1], %[c]"
-        : [r0] "+v"(r0), [r1] "+v"(r1), [t0] "=&v"(t0), [t1] "=&v"(t1), [b] "=&s"(b), [m] "=&s"(m), [c] "+s"(c)
-        : [x3] "v"(x.x3)
+        "v_cndmask_b32_e64 %[x3], 0, -1, %[m]\n\t"
+        "v_addc_co_u32_e64 %[r0], %[c], %[r0], %[x3], %[b]\n\t"
+        "v_cndmask_b32_e64 %[x3], 0, -1, %[b]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32_e64 %[r1], %[c], %[r1], %[x3], %[c]"
+        : [r0] "+v"(r0), [r1] "+v"(r1), [x3] "+v"(x3), [b] "=&s"(b), [m] "=&s"(m), [c] "+s"(c)
+        :
         : "scc");
     return gl_pack(r0, r1);
 }
@@ -266,34 +264,35 @@ __device__ __forceinline__ void gl_reducek3(const gl_prodk *x, uint64_t *out)
 
 // One lane of gl_prodk3 / gl_reducek3, the gaps that no instruction fills taken by s_nop:
 // k is read three multiply-adds after its write, and scalar instructions wait for a mask
-// that a vector instruction writes by themselves.
+// that a vector instruction writes by themselves. The vector registers it writes are those
+// of its operands, here and in gl_mulk2 and gl_prod_reduce1 (gl_digits.h, wait states).
 template <bool BU = false>
 __device__ __forceinline__ uint64_t gl_mulk1(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi)
 {
     uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32), b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
     uint64_t p = (uint64_t)a0 * b0 + s_lo;
     uint64_t t = (uint64_t)a0 * b1 + ((p >> 32) + (uint64_t)s_hi);
-    uint64_t u, k;
+    uint64_t u = t, k;
     if constexpr (BU)
-        asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=&v"(u), "=&s"(k) : "v"(a1), "s"(b0), "v"(t));
+        asm("v_mad_u64_u32 %0, %1, %2, %3, %0" : "+v"(u), "=s"(k) : "v"(a1), "s"(b0));
     else
-        asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=&v"(u), "=&s"(k) : "v"(a1), "v"(b0), "v"(t));
+        asm("v_mad_u64_u32 %0, %1, %2, %3, %0" : "+v"(u), "=s"(k) : "v"(a1), "v"(b0));
     uint64_t h = (uint64_t)a1 * b1 + (u >> 32);
-    uint64_t lo = gl_pack((uint32_t)p, (uint32_t)u), r, c, bm, m;
-    asm("v_mad_u64_u32 %0, %1, %2, -1, %3" : "=&v"(r), "=&s"(c) : "v"((uint32_t)h), "v"(lo));
-    uint32_t r0 = (uint32_t)r, r1 = (uint32_t)(r >> 32), tm, tn;
+    uint64_t r = gl_pack((uint32_t)p, (uint32_t)u), c, bm, m;
+    asm("v_mad_u64_u32 %0, %1, %2, -1, %0" : "+v"(r), "=s"(c) : "v"((uint32_t)h));
+    uint32_t r0 = (uint32_t)r, r1 = (uint32_t)(r >> 32), x3 = (uint32_t)(h >> 32);
     asm("v_subb_co_u32_e64 %[r0], %[b], %[r0], %[x3], %[k]\n\t"
         "s_nop 1\n\t"
         "v_subb_co_u32_e64 %[r1], %[b], %[r1], 0, %[b]\n\t"
         "s_andn2_b64 %[m], %[c], %[b]\n\t"
         "s_andn2_b64 %[b], %[b], %[c]\n\t"
-        "v_cndmask_b32_e64 %[tm], 0, -1, %[m]\n\t"
-        "v_cndmask_b32_e64 %[tn], 0, -1, %[b]\n\t"
-        "v_addc_co_u32_e64 %[r0], %[c], %[r0], %[tm], %[b]\n\t"
-        "s_nop 1\n\t"
-        "v_addc_co_u32_e64 %[r1], %[c], %[r1], %[tn], %[c]"
-        : [r0] "+v"(r0), [r1] "+v"(r1), [tm] "=&v"(tm), [tn] "=&v"(tn), [b] "=&s"(bm), [m] "=&s"(m), [c] "+s"(c)
-        : [x3] "v"((uint32_t)(h >> 32)), [k] "s"(k)
+        "v_cndmask_b32_e64 %[x3], 0, -1, %[m]\n\t"
+        "v_addc_co_u32_e64 %[r0], %[c], %[r0], %[x3], %[b]\n\t"
+        "v_cndmask_b32_e64 %[x3], 0, -1, %[b]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32_e64 %[r1], %[c], %[r1], %[x3], %[c]"
+        : [r0] "+v"(r0), [r1] "+v"(r1), [x3] "+v"(x3), [b] "=&s"(bm), [m] "=&s"(m), [c] "+s"(c)
+        : [k] "s"(k)
         : "scc");
     return gl_pack(r0, r1);
 }
@@ -302,29 +301,30 @@ __device__ __forceinline__ uint64_t gl_mulk1(uint64_t a, uint64_t b, uint32_t s_
 // one's gaps (one wait state is left to s_nop).
 __device__ __forceinline__ void gl_mulk2(const uint64_t *a, const uint64_t *b, uint64_t *out)
 {
-    uint64_t p[2], t[2], u[2], k[2], h[2], r[2], c[2], bm[2], m[2];
-    uint32_t r0[2], r1[2], tm[2], tn[2];
+    uint64_t p[2], u[2], k[2], h[2], r[2], c[2], bm[2], m[2];
+    uint32_t r0[2], r1[2], x3[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         p[i] = (uint64_t)(uint32_t)a[i] * (uint32_t)b[i];
-        t[i] = (uint64_t)(uint32_t)a[i] * (uint32_t)(b[i] >> 32) + (p[i] >> 32);
+        u[i] = (uint64_t)(uint32_t)a[i] * (uint32_t)(b[i] >> 32) + (p[i] >> 32);
     }
-    asm("v_mad_u64_u32 %0, %2, %4, %6, %8\n\t"
-        "v_mad_u64_u32 %1, %3, %5, %7, %9"
-        : "=&v"(u[0]), "=&v"(u[1]), "=&s"(k[0]), "=&s"(k[1])
-        : "v"((uint32_t)(a[0] >> 32)), "v"((uint32_t)(a[1] >> 32)), "v"((uint32_t)b[0]), "v"((uint32_t)b[1]), "v"(t[0]),
-          "v"(t[1]));
+    asm("v_mad_u64_u32 %0, %2, %4, %6, %0\n\t"
+        "v_mad_u64_u32 %1, %3, %5, %7, %1"
+        : "+&v"(u[0]), "+&v"(u[1]), "=&s"(k[0]), "=&s"(k[1])
+        : "v"((uint32_t)(a[0] >> 32)), "v"((uint32_t)(a[1] >> 32)), "v"((uint32_t)b[0]), "v"((uint32_t)b[1]));
 #pragma unroll
     for (int i = 0; i < 2; i++) h[i] = (uint64_t)(uint32_t)(a[i] >> 32) * (uint32_t)(b[i] >> 32) + (u[i] >> 32);
-    asm("v_mad_u64_u32 %0, %2, %4, -1, %6\n\t"
-        "v_mad_u64_u32 %1, %3, %5, -1, %7"
-        : "=&v"(r[0]), "=&v"(r[1]), "=&s"(c[0]), "=&s"(c[1])
-        : "v"((uint32_t)h[0]), "v"((uint32_t)h[1]), "v"(gl_pack((uint32_t)p[0], (uint32_t)u[0])),
-          "v"(gl_pack((uint32_t)p[1], (uint32_t)u[1])));
+#pragma unroll
+    for (int i = 0; i < 2; i++) r[i] = gl_pack((uint32_t)p[i], (uint32_t)u[i]);
+    asm("v_mad_u64_u32 %0, %2, %4, -1, %0\n\t"
+        "v_mad_u64_u32 %1, %3, %5, -1, %1"
+        : "+&v"(r[0]), "+&v"(r[1]), "=&s"(c[0]), "=&s"(c[1])
+        : "v"((uint32_t)h[0]), "v"((uint32_t)h[1]));
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         r0[i] = (uint32_t)r[i];
         r1[i] = (uint32_t)(r[i] >> 32);
+        x3[i] = (uint32_t)(h[i] >> 32);
     }
     asm("v_subb_co_u32_e64 %[r0a], %[ba], %[r0a], %[x3a], %[ka]\n\t"
         "v_subb_co_u32_e64 %[r0b], %[bb], %[r0b], %[x3b], %[kb]\n\t"
@@ -335,18 +335,18 @@ __device__ __forceinline__ void gl_mulk2(const uint64_t *a, const uint64_t *b, u
         "s_andn2_b64 %[ba], %[ba], %[ca]\n\t"
         "s_andn2_b64 %[mb], %[cb], %[bb]\n\t"
         "s_andn2_b64 %[bb], %[bb], %[cb]\n\t"
-        "v_cndmask_b32_e64 %[tma], 0, -1, %[ma]\n\t"
-        "v_cndmask_b32_e64 %[tmb], 0, -1, %[mb]\n\t"
-        "v_addc_co_u32_e64 %[r0a], %[ca], %[r0a], %[tma], %[ba]\n\t"
-        "v_addc_co_u32_e64 %[r0b], %[cb], %[r0b], %[tmb], %[bb]\n\t"
-        "v_cndmask_b32_e64 %[tma], 0, -1, %[ba]\n\t"
-        "v_cndmask_b32_e64 %[tmb], 0, -1, %[bb]\n\t"
-        "v_addc_co_u32_e64 %[r1a], %[ca], %[r1a], %[tma], %[ca]\n\t"
-        "v_addc_co_u32_e64 %[r1b], %[cb], %[r1b], %[tmb], %[cb]"
-        : [r0a] "+v"(r0[0]), [r0b] "+v"(r0[1]), [r1a] "+v"(r1[0]), [r1b] "+v"(r1[1]), [tma] "=&v"(tm[0]),
-          [tmb] "=&v"(tm[1]), [ba] "=&s"(bm[0]), [bb] "=&s"(bm[1]), [ma] "=&s"(m[0]), [mb] "=&s"(m[1]), [ca] "+s"(c[0]),
+        "v_cndmask_b32_e64 %[x3a], 0, -1, %[ma]\n\t"
+        "v_cndmask_b32_e64 %[x3b], 0, -1, %[mb]\n\t"
+        "v_addc_co_u32_e64 %[r0a], %[ca], %[r0a], %[x3a], %[ba]\n\t"
+        "v_addc_co_u32_e64 %[r0b], %[cb], %[r0b], %[x3b], %[bb]\n\t"
+        "v_cndmask_b32_e64 %[x3a], 0, -1, %[ba]\n\t"
+        "v_cndmask_b32_e64 %[x3b], 0, -1, %[bb]\n\t"
+        "v_addc_co_u32_e64 %[r1a], %[ca], %[r1a], %[x3a], %[ca]\n\t"
+        "v_addc_co_u32_e64 %[r1b], %[cb], %[r1b], %[x3b], %[cb]"
+        : [r0a] "+v"(r0[0]), [r0b] "+v"(r0[1]), [r1a] "+v"(r1[0]), [r1b] "+v"(r1[1]), [x3a] "+v"(x3[0]),
+          [x3b] "+v"(x3[1]), [ba] "=&s"(bm[0]), [bb] "=&s"(bm[1]), [ma] "=&s"(m[0]), [mb] "=&s"(m[1]), [ca] "+s"(c[0]),
           [cb] "+s"(c[1])
-        : [x3a] "v"((uint32_t)(h[0] >> 32)), [x3b] "v"((uint32_t)(h[1] >> 32)), [ka] "s"(k[0]), [kb] "s"(k[1])
+        : [ka] "s"(k[0]), [kb] "s"(k[1])
         : "scc");
     out[0] = gl_pack(r0[0], r1[0]);
     out[1] = gl_pack(r0[1], r1[1]);

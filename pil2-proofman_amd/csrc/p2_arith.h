@@ -122,8 +122,8 @@ __device__ __forceinline__ void hz_fold3(const hz *a, uint64_t *out)
 // One halves-form fold (hz_fold3's steps, hazard gaps filled with s_nop).
 __device__ __forceinline__ uint64_t hz_fold(hz a)
 {
-    uint64_t r, d, c;
-    asm("v_mad_u64_u32 %0, %1, %2, -1, %3" : "=&v"(r), "=&s"(d) : "v"((uint32_t)(a.hi >> 32)), "v"(a.lo));
+    uint64_t r = a.lo, d, c;
+    asm("v_mad_u64_u32 %0, %1, %2, -1, %0" : "+v"(r), "=s"(d) : "v"((uint32_t)(a.hi >> 32)));
     uint32_t r0 = (uint32_t)r, r1 = (uint32_t)(r >> 32);
     uint64_t b;
     asm("v_add_co_u32_e64 %[r1], %[c], %[r1], %[h0]\n\t"
@@ -140,11 +140,11 @@ __device__ __forceinline__ uint64_t hz_fold(hz a)
 // Two halves-form folds in step
 __device__ __forceinline__ void hz_fold2(const hz *a, uint64_t *out)
 {
-    uint64_t r[2], d[2], c[2], bb[2];
-    asm("v_mad_u64_u32 %0, %2, %4, -1, %6\n\t"
-        "v_mad_u64_u32 %1, %3, %5, -1, %7"
-        : "=&v"(r[0]), "=&v"(r[1]), "=&s"(d[0]), "=&s"(d[1])
-        : "v"((uint32_t)(a[0].hi >> 32)), "v"((uint32_t)(a[1].hi >> 32)), "v"(a[0].lo), "v"(a[1].lo));
+    uint64_t r[2] = {a[0].lo, a[1].lo}, d[2], c[2], bb[2];
+    asm("v_mad_u64_u32 %0, %2, %4, -1, %0\n\t"
+        "v_mad_u64_u32 %1, %3, %5, -1, %1"
+        : "+&v"(r[0]), "+&v"(r[1]), "=&s"(d[0]), "=&s"(d[1])
+        : "v"((uint32_t)(a[0].hi >> 32)), "v"((uint32_t)(a[1].hi >> 32)));
     uint32_t r0[2], r1[2];
 #pragma unroll
     for (int k = 0; k < 2; k++) {

@@ -191,27 +191,14 @@ __device__ __forceinline__ p2_rows p2_operand_rows(const p2_v4i *s)
 }
 
 // The result whose eight digit sums (absolute values < 2^22) start at acc[at]: lo + 2^32 hi
-// plus the addends k, the same for the wave or (p2_digits_v) each lane's own
-#define P2_DIGITS(NAME, KC)                                                                           \
-    __device__ __forceinline__ hz NAME(const p2_v16i &acc, int at, const uint64_t *k, uint32_t c16)   \
-    {                                                                                                 \
-        uint32_t e[4];                                                                                \
-        _Pragma("unroll") for (int i = 0; i < 4; i++) e[i] =                                          \
-            ((uint32_t)acc[at + 2 * i + 1] << 8) + (uint32_t)acc[at + 2 * i];                         \
-        uint64_t l, h, d0, d1;                                                                        \
-        asm("v_mad_i64_i32 %0, %2, %4, %6, %7\n\t"                                                    \
-            "v_mad_i64_i32 %1, %3, %5, %6, %8"                                                        \
-            : "=&v"(l), "=&v"(h), "=&s"(d0), "=&s"(d1)                                                \
-            : "v"(e[1]), "v"(e[3]), "v"(c16), KC(k[0]), KC(k[1]));                                    \
-        hz r;                                                                                         \
-        asm("v_mad_i64_i32 %0, %2, %4, 1, %6\n\t"                                                     \
-            "v_mad_i64_i32 %1, %3, %5, 1, %7"                                                         \
-            : "=&v"(r.lo), "=&v"(r.hi), "=&s"(d0), "=&s"(d1)                                          \
-            : "v"(e[0]), "v"(e[2]), "v"(l), "v"(h));                                                  \
-        return r;                                                                                     \
-    }
-P2_DIGITS(p2_digits, "s")
-P2_DIGITS(p2_digits_v, "v")
+// plus the addends k, the same for the wave (SK) or each lane's own
+template <bool SK>
+__device__ __forceinline__ hz p2_digits(const p2_v16i &acc, int at, const uint64_t *k)
+{
+    const gl_v4i a = {acc[at], acc[at + 1], acc[at + 2], acc[at + 3]};
+    const gl_v4i b = {acc[at + 4], acc[at + 5], acc[at + 6], acc[at + 7]};
+    return gl_digit_sums<SK>(a, b, k[0], k[1]);
+}
 
 // The A operands on their way from LDS, P2_AHEAD of them (1 and 2 measure the same within
 // 2 %; more pushes width 16 further over 128 VGPRs). First those of the u, then the state's.
@@ -269,7 +256,6 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int 
     using Op = p2c::Operands<W>;
     constexpr int NS = Op::NS, NY = Op::NY, NU = Op::NU;
     const uint64_t(*k)[2] = c_p2_addends<W>.k[g];
-    const uint32_t c16 = 65536;
     p2_v4i in[2 * Op::NK];
     p2_stream<W> st;
     st.start(ops);
@@ -282,7 +268,7 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int 
     st.mac(acc, in[NS - 1]);
 #pragma unroll
     for (int p = 0; p < NU; p++) {
-        hz u = p2_digits(acc, 0, k[2 * p], c16);
+        hz u = p2_digits<true>(acc, 0, k[2 * p]);
         nxt = (p2_v16i){};
 #pragma unroll
         for (int t = 0; t < NS + p && p + 1 < NU; t++) st.mac(nxt, in[t]);
@@ -290,7 +276,7 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int 
         gl_put_word(in[NS + p], 0, y);
         gl_put_word(in[NS + p], 1, y);  // any value: its coefficients in the next operand are zero
         st.mac(acc, in[NS + p]);
-        u = p2_digits(acc, 8, k[2 * p + 1], c16);
+        u = p2_digits<true>(acc, 8, k[2 * p + 1]);
         // the first word's sums are written again by the second product: they stay
         // reserved until its results have been read
         asm volatile("" : "+v"(u.lo) : "v"(acc));
@@ -318,8 +304,8 @@ __device__ __forceinline__ void p2_segment(uint64_t *s, const p2_rows &ops, int 
         for (int t = 0; t < Op::NK; t++) st.mac2(acc, in[2 * t], nxt, in[2 * t + 1]);
 #pragma unroll
         for (int o = 0; o < 2; o++) {
-            uint64_t x = hz_fold(p2_digits_v(acc, 8 * o, kh[4 * m + o], c16));
-            uint64_t y = hz_fold(p2_digits_v(nxt, 8 * o, kh[4 * m + o], c16));
+            uint64_t x = hz_fold(p2_digits<false>(acc, 8 * o, kh[4 * m + o]));
+            uint64_t y = hz_fold(p2_digits<false>(nxt, 8 * o, kh[4 * m + o]));
             asm volatile("s_nop 1" : "+v"(x), "+v"(y));  // the exchange reads what inline assembly wrote
             int x0 = (int)(uint32_t)x, x1 = (int)(x >> 32), y0 = (int)(uint32_t)y, y1 = (int)(y >> 32);
             p2_swap32(x0, y0);
