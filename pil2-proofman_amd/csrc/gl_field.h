@@ -263,8 +263,10 @@ __device__ __forceinline__ void gl_reducek3(const gl_prodk *x, uint64_t *out)
 }
 
 // One lane of gl_prodk3 / gl_reducek3, the gaps that no instruction fills taken by s_nop:
-// k is read three multiply-adds after its write, and scalar instructions wait for a mask
-// that a vector instruction writes by themselves. The vector registers it writes are those
+// between the write of k and its read stand the move of u's low word to the high register of
+// the pair lo (pairs start at even registers, so it is always a move) and the multiply-add
+// of r, and with them that of h where no half of a factor is known to be zero; scalar
+// instructions wait for a mask that a vector instruction writes by themselves. The vector registers it writes are those
 // of its operands, here and in gl_mulk2 and gl_prod_reduce1 (gl_digits.h, wait states).
 template <bool BU = false>
 __device__ __forceinline__ uint64_t gl_mulk1(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi)

@@ -150,3 +150,47 @@ def test_matrix_registers_are_not_overwritten_early(code):
     assert len(matrix) > 40
     bad = ["%s: %s" % (f, h) for f in matrix for h in matrix_hazards(code[f])]
     assert not bad, "%d early accesses:\n%s" % (len(bad), "\n".join(bad[:20]))
+
+
+# VALU instructions between a VALU write of scalar registers (a carry mask) and a VALU
+# read of them
+MASK_WAIT = 2
+
+
+def mask_hazards(code):
+    out, at = [], {i.address: k for k, i in enumerate(code)}
+    for k, i in enumerate(code):
+        masks = {r for r in i.writes if r[0] == "s"}
+        if masks:
+            out += early(code, at, k, [("mask", masks, MASK_WAIT, False, True)])
+    return out
+
+
+def test_carry_masks_are_not_read_early(code):
+    bad = ["%s: %s" % (f, h) for f, c in code.items() for h in mask_hazards(c)]
+    assert not bad, "%d early reads:\n%s" % (len(bad), "\n".join(bad[:20]))
+
+
+# Factors whose halves the compiler knows in part, so that it leaves out a multiply-add of
+# the chain that the masks' distances are counted in
+KNOWN = ["(uint64_t)(uint32_t)a[i]", "a[i] << 32", "7", "0x7000000000000000ull"]
+PRODUCTS = ["gl_mulk1(x, {f}, 0, 0)", "gl_mulk1({f}, x, 0, 0)", "gl_mulk1({f}, {f}, 0, 0)", "gl_mulk1(x, {f}, k, k)",
+            "gl_mul(x, {f})", "gl_mul({f}, {f})", "gl_mul_nc(x, {f})"]
+
+
+def test_products_by_known_factors_keep_the_distance(tmp_path):
+    import build
+    calls = [p.format(f=f) for p in PRODUCTS for f in KNOWN]
+    calls += ["gl_mulk1<true>(x, %s, 0, 0)" % f for f in ("(uint64_t)k", "(uint64_t)k << 32", "7")]
+    src, obj = tmp_path / "k.hip", tmp_path / "k.co"
+    src.write_text('#include "gl_field.h"\n' + "".join(
+        'extern "C" __global__ void k%d(uint64_t *a, uint32_t k)\n{\n    const int i = threadIdx.x;\n'
+        "    const uint64_t x = a[i + 64];\n    a[i] = %s;\n}\n" % (n, c) for n, c in enumerate(calls)))
+    subprocess.run(["hipcc"] + build.FLAGS + ["-w", "--offload-device-only", "--no-gpu-bundle-output", "-c", "-I",
+                                              build.CSRC, str(src), "-o", str(obj)], check=True, capture_output=True)
+    text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(obj)], check=True, capture_output=True,
+                          text=True).stdout
+    kernels = functions(text)
+    assert set(kernels) == {"k%d" % n for n in range(len(calls))}
+    bad = {c: mask_hazards(kernels["k%d" % n]) for n, c in enumerate(calls)}
+    assert not any(bad.values()), {c: h for c, h in bad.items() if h}
