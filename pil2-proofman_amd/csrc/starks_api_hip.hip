@@ -1337,6 +1337,12 @@ static int64_t fri_branch_resources(uint64_t layers)
     return 0;
 }
 
+// Whether na words at a and nb words at b share any
+static bool overlap(const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb)
+{
+    return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
 // branches: each layer's tree goes on branch stream (layer mod kFriBranches),
 // forked from st after the layer's transpose and joined into st at the end (used
 // under graph capture, where the fork and join become graph edges).
@@ -1350,7 +1356,10 @@ static int64_t fri_enqueue(const uint64_t *d_pol, uint64_t *d_work, const uint64
     for (uint64_t s = 0; s < n && !rc; s++) {
         // The fold writes a short layer's tree source itself: the next fold, in place, then
         // waits for no transpose. A long layer's rows would be written in pieces of 24 bytes.
-        const bool fused = s > 0 && s + 1 < n && steps[s] <= kFriFusedBits;
+        // A source within what the fold reads (d_pol after its last use, the rest of d_work)
+        // is written after it.
+        const bool fused = s > 0 && s + 1 < n && steps[s] <= kFriFusedBits &&
+                           !overlap(d_sources[s], 3ull << steps[s], s == 1 ? d_pol : d_work, 3ull << steps[s - 1]);
         if (s > 0) {
             int e = fri_launch_fold2(d_work, s == 1 ? d_pol : d_work, nullptr, d_ch + 3 * s, nbe, steps[s - 1],
                                      steps[s], fri_tables(st), fused ? d_sources[s] : nullptr,
