@@ -45,12 +45,12 @@ extern "C" int ntt_launch_compute_q(uint64_t *cmq, const uint64_t *q, uint64_t q
                                     uint32_t log_n, uint32_t log_ext, uint32_t q_deg, uint32_t q_dim,
                                     const NttTablesHost *th, hipStream_t st);
 // NTT / INTT of M = 2^lm >= 16 rows (natural order; the inverse includes 1/M) in two steps.
-// Bit reversal (and 1/M), out of place: of columns, or of rows into columns (tmp: M * ncols
-// words, used with long, narrow data)
+// Bit reversal (and 1/M), out of place: of columns, or of rows into columns. The latter are
+// in a (M * ncols words), or with long, narrow data by way of a in b (*out); src may lie in b
 extern "C" int ntt_launch_bitrev(uint64_t *out, const uint64_t *src, uint32_t lm, uint64_t ncols, int inverse,
                                  hipStream_t st);
-extern "C" int ntt_launch_bitrev_rows(uint64_t *out, uint64_t *tmp, const uint64_t *src, uint32_t lm, uint64_t ncols,
-                                      int inverse, hipStream_t st);
+extern "C" int ntt_launch_bitrev_rows(uint64_t *a, uint64_t *b, uint64_t **out, const uint64_t *src, uint32_t lm,
+                                      uint64_t ncols, int inverse, hipStream_t st);
 // The transform of bit-reversed columns; dst may equal src
 extern "C" int ntt_launch_reversed(uint64_t *dst, const uint64_t *src, uint32_t lm, uint64_t ncols, int inverse,
                                    const NttTablesHost *th, hipStream_t st);

@@ -1330,17 +1330,18 @@ extern "C" int ntt_launch_bitrev(uint64_t *out, const uint64_t *src, uint32_t lm
     return (int)hipGetLastError();
 }
 
-extern "C" int ntt_launch_bitrev_rows(uint64_t *out, uint64_t *tmp, const uint64_t *src, uint32_t lm, uint64_t ncols,
-                                      int inverse, hipStream_t st)
+extern "C" int ntt_launch_bitrev_rows(uint64_t *a, uint64_t *b, uint64_t **out, const uint64_t *src, uint32_t lm,
+                                      uint64_t ncols, int inverse, hipStream_t st)
 {
     uint64_t M = 1ull << lm;
+    *out = transpose_bitrev(lm, ncols) ? a : b;
     if (lm < 4 || lm > NTT_MAX_LOG) return -3;
-    if (!transpose_bitrev(lm, ncols)) {
-        int e = ntt_launch_rm2cm(tmp, src, M, ncols, ncols, M, st);
-        return e ? e : ntt_launch_bitrev(out, tmp, lm, ncols, inverse, st);
+    if (*out == b) {
+        int e = ntt_launch_rm2cm(a, src, M, ncols, ncols, M, st);
+        return e ? e : ntt_launch_bitrev(b, a, lm, ncols, inverse, st);
     }
     dim3 g((unsigned)((M + TRB_ROWS - 1) / TRB_ROWS), (unsigned)((ncols + TRB_COLS - 1) / TRB_COLS));
-    hipLaunchKernelGGL(k_transpose_bitrev, g, dim3(256), 0, st, src, out, lm, ncols, inverse ? gl_inv(M % GL_P) : 1);
+    hipLaunchKernelGGL(k_transpose_bitrev, g, dim3(256), 0, st, src, a, lm, ncols, inverse ? gl_inv(M % GL_P) : 1);
     return (int)hipGetLastError();
 }
 

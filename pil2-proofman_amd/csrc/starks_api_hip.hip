@@ -536,6 +536,12 @@ int64_t pil2hip_commit_host(uint64_t *d_lde, uint64_t *d_nodes, const uint64_t *
     return 0;
 }
 
+// Whether na words at a and nb words at b share any
+static bool overlap(const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb)
+{
+    return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
 int64_t pil2hip_ntt(uint64_t *d_dst, const uint64_t *d_src, uint64_t *d_scratch, uint64_t nBits, uint64_t nCols,
                     bool inverse, bool rowMajor, void *stream)
 {
@@ -556,10 +562,13 @@ int64_t pil2hip_ntt(uint64_t *d_dst, const uint64_t *d_src, uint64_t *d_scratch,
         if (rc) return rc;
         if (rowMajor) {  // rows -> bit-reversed columns, transform, columns -> rows
             if (!d_scratch) return fail(-13, "row-major transforms need a scratch of 2 * 2^nBits * nCols words");
-            uint64_t *a = d_scratch, *b = d_scratch + M * nCols;
-            e = ntt_launch_bitrev_rows(a, b, d_src, (uint32_t)nBits, nCols, inverse, st);
-            if (!e) e = ntt_launch_reversed(a, a, (uint32_t)nBits, nCols, inverse, tb, st);
-            if (!e) e = ntt_launch_cm2rm(d_dst, a, M, nCols, M, nCols, st);
+            // d_dst may lie in a half of the scratch, d_src in the second one
+            const uint64_t words = M * nCols;
+            uint64_t *a = d_scratch, *b = d_scratch + words, *from;
+            e = ntt_launch_bitrev_rows(a, b, &from, d_src, (uint32_t)nBits, nCols, inverse, st);
+            uint64_t *to = overlap(d_dst, words, from, words) ? (from == a ? b : a) : from;
+            if (!e) e = ntt_launch_reversed(to, from, (uint32_t)nBits, nCols, inverse, tb, st);
+            if (!e) e = ntt_launch_cm2rm(d_dst, to, M, nCols, M, nCols, st);
         } else if (d_dst == d_src) {
             if (!d_scratch) return fail(-13, "in-place column-major transforms need a scratch of 2^nBits * nCols words");
             e = ntt_launch_bitrev(d_scratch, d_src, (uint32_t)nBits, nCols, inverse, st);
@@ -1335,12 +1344,6 @@ static int64_t fri_branch_resources(uint64_t layers)
         g_fri_fork.push_back(e);
     }
     return 0;
-}
-
-// Whether na words at a and nb words at b share any
-static bool overlap(const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb)
-{
-    return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
 }
 
 // branches: each layer's tree goes on branch stream (layer mod kFriBranches),

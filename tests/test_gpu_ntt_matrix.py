@@ -112,3 +112,27 @@ def test_ntt_rows_long(pc, lg, cols):
     ntt.INTT(None, columns, n, cols, row_major=False)
     torch.cuda.synchronize()
     assert torch.equal(rows.reshape(n, cols), columns.reshape(cols, n).t())
+
+
+@pytest.mark.parametrize("lg,cols", [(4, 3), (7, 40), (10, 17), (15, 5), (23, 3)])
+@pytest.mark.parametrize("dst_half,src_half", [(0, None), (1, None), (None, 1), (0, 1), (1, 1)])
+def test_ntt_rows_within_the_scratch(pc, lg, cols, dst_half, src_half):
+    """Row-major data whose result lies in a half of the scratch, or whose source lies in the
+    second half: as with buffers of their own."""
+    import torch
+    n = 1 << lg
+    raw, _ = _words(n * cols, 8600 + lg)
+    ntt = pc.NTT_Goldilocks(n)
+    want = pc.empty(n * cols)
+    ntt.NTT(want, pc.to_device(raw), n, cols, row_major=True)
+    buffer = pc.empty(2 * n * cols)
+    src, dst = pc.to_device(raw), pc.empty(n * cols)
+    if src_half is not None:
+        half = buffer[src_half * n * cols:(src_half + 1) * n * cols]
+        half.copy_(src)
+        src = half
+    if dst_half is not None:
+        dst = buffer[dst_half * n * cols:(dst_half + 1) * n * cols]
+    ntt.NTT(dst, src, n, cols, buffer=buffer, row_major=True)
+    torch.cuda.synchronize()
+    assert torch.equal(dst, want)
