@@ -136,3 +136,42 @@ def test_ntt_rows_within_the_scratch(pc, lg, cols, dst_half, src_half):
     ntt.NTT(dst, src, n, cols, buffer=buffer, row_major=True)
     torch.cuda.synchronize()
     assert torch.equal(dst, want)
+
+
+# blocks of two columns: even pairs and an odd last column, every line of a piece its own
+# (blowup 8) or shared by waves (blowup 4), and one column fewer than pairs begin with
+PAIRS = [(19, 3, 32), (19, 3, 33), (19, 3, 31), (20, 3, 16), (20, 3, 17), (21, 3, 8), (21, 3, 9), (20, 2, 32), (20, 2, 33),
+         (21, 2, 17), (22, 2, 9)]
+
+
+@pytest.mark.parametrize("nb,lb,cols", PAIRS)
+def test_lde_in_pairs(pc, oracle, nb, lb, cols):
+    import torch
+    n, ne = 1 << nb, 1 << (nb + lb)
+    some = sorted({0, 1, cols // 2 | 1, cols - 2, cols - 1})
+    trace = pc.fill_uniform(pc.empty(n * cols), 7100 + 40 * nb + cols).reshape(n, cols)
+    raw = pc.to_host(trace[:, some].contiguous()).reshape(n, len(some)).copy()
+    edge, _ = _words(len(some) * 1000, 7200 + cols)
+    raw[:1000] = edge.reshape(1000, len(some))
+    trace[:, some] = pc.to_device(raw)
+    out = pc.empty(ne * cols)
+    pc.NTT_Goldilocks(n).LDE(out, trace, ne, n, cols)
+    torch.cuda.synchronize()
+    want = oracle.lde(np.where(raw >= np.uint64(P), raw - np.uint64(P), raw), ne)
+    got = out.reshape(cols, ne)
+    for k, c in enumerate(some):
+        assert (pc.to_host(got[c]) == want[:, k]).all(), c
+
+
+@pytest.mark.parametrize("lg", [23, 24])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_ntt_longest_strided(pc, oracle, lg, inverse):
+    """The transforms with 9 and 10 bits in the strided pass."""
+    import torch
+    n = 1 << lg
+    raw, a = _words(n, 8000 + lg)
+    d = pc.to_device(raw)
+    ntt = pc.NTT_Goldilocks(n)
+    (ntt.INTT if inverse else ntt.NTT)(None, d, n, 1, row_major=False)
+    torch.cuda.synchronize()
+    assert (pc.to_host(d) == (oracle.intt if inverse else oracle.ntt)(a)).all()
