@@ -215,3 +215,38 @@ def test_batch_plan_defaults_and_errors(pc):
                 pc.Pil2CommitPlan(17, 0, 0, 0)):
         assert pc.lib.pil2hip_commit_batch_plan(pc.ctypes.cast(b._arr, pc._vp), len(b.jobs), pc.ctypes.byref(bad),
                                                 None, pc._ptr(b.roots), pc._stream()) < 0
+
+
+# transforms whose rounds stay on the VALU, so that the plan's tile and radix count: blowup 16
+# with 4 to 9 strided bits, one block of each blowup below 2^10 values, and above 2^24 rows
+VALU_SHAPES = [(14, 18, 2), (16, 20, 1), (18, 22, 3), (12, 16, 5), (9, 13, 2), (6, 8, 3), (8, 9, 2), (24, 25, 1)]
+
+
+def _signature(pc, nb, nbe, plan):
+    class NttPlan(pc.ctypes.Structure):
+        _fields_ = [("tile_log", pc.ctypes.c_uint32), ("radix_log", pc.ctypes.c_uint32)]
+
+    f = pc.lib.ntt_lde_plan_signature
+    f.restype = pc.ctypes.c_uint64
+    return f(nb, nbe, pc.ctypes.byref(NttPlan(plan["ntt_tile_log"], plan["ntt_radix_log"])))
+
+
+def test_batch_plans_of_valu_transforms(pc, oracle):
+    """The plans of test_batch_plans_are_bit_identical on shapes whose launches they change."""
+    for nb, nbe, _ in VALU_SHAPES:
+        assert len({_signature(pc, nb, nbe, p) for p in PLANS}) >= (3 if nb < 9 else len(PLANS)), (nb, nbe)
+    jobs = _jobs(pc, VALU_SHAPES, 5252)
+    want = [_plain(pc, j, 3) for j in jobs]
+    for j, (nb, nbe, nc), (lde, nodes) in zip(jobs[:-1], VALU_SHAPES, want):
+        trace = pc.to_host(j["trace"]).reshape(1 << nb, nc)
+        ref = oracle.lde(trace, 1 << nbe)
+        assert np.array_equal(lde.reshape(nc, 1 << nbe).T, ref), (nb, nbe)
+        assert np.array_equal(nodes[-4:], oracle.merkletree(ref, 3)[-4:]), (nb, nbe)
+    for plan in PLANS:
+        print("plan", plan, flush=True)
+        b = pc.CommitBatch(jobs, arity=3)
+        assert b.launch(plan=plan) == plan["n_streams"]
+        _sync()
+        for k, j in enumerate(b.jobs):
+            assert np.array_equal(pc.to_host(j["lde"]), want[k][0]), (plan, "lde", k)
+            assert np.array_equal(pc.to_host(j["nodes"]), want[k][1]), (plan, "nodes", k)
