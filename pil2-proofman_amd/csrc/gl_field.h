@@ -1279,13 +1279,6 @@ __host__ __device__ __forceinline__ uint64_t gl_inv(uint64_t a) { return gl_pow(
 // F_p[x]/(x^3 - x - 1), element = (c0, c1, c2) stored interleaved as 3 u64.
 struct gl3 { uint64_t v[3]; };
 
-__host__ __device__ __forceinline__ gl3 gl3_add(const gl3 &a, const gl3 &b)
-{
-    gl3 r;
-    for (int k = 0; k < 3; k++) r.v[k] = gl_add(a.v[k], b.v[k]);
-    return r;
-}
-
 // Karatsuba-style product with x^3 = x + 1 (goldilocks_cubic_extension.hpp:232-245)
 __host__ __device__ __forceinline__ gl3 gl3_mul(const gl3 &a, const gl3 &b)
 {

@@ -174,13 +174,7 @@ __device__ __forceinline__ uint64_t p2_mul(uint64_t a, uint64_t b) { return gl_m
 // two of them in step
 __device__ __forceinline__ void p2_mul2(const uint64_t *a, const uint64_t *b, uint64_t *out) { gl_mulk2(a, b, out); }
 
-// a*b + s mod p as a 64-bit word (s = s_hi:s_lo)
-__device__ __forceinline__ uint64_t p2_mul_add(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi)
-{
-    return gl_mulk1(a, b, s_lo, s_hi);
-}
-
-// p2_mul_add with a wave-uniform b
+// a*b + s mod p as a 64-bit word (s = s_hi:s_lo), b wave-uniform
 __device__ __forceinline__ uint64_t p2_mul_add_u(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi)
 {
     return gl_mulk1<true>(a, b, s_lo, s_hi);
@@ -214,7 +208,6 @@ __device__ void hz_fold2(const hz *a, uint64_t *out);
 __device__ uint64_t lz_fold(lz a);
 __device__ uint64_t p2_mul(uint64_t a, uint64_t b);
 __device__ void p2_mul2(const uint64_t *a, const uint64_t *b, uint64_t *out);
-__device__ uint64_t p2_mul_add(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi);
 __device__ uint64_t p2_mul_add_u(uint64_t a, uint64_t b, uint32_t s_lo, uint32_t s_hi);
 
 #endif

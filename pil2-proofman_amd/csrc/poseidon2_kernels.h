@@ -3,7 +3,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#define P2_THREADS 256
 // tree levels with at most this many parents use 16 lanes per permutation (default)
 #ifndef P2_COOP_MAX_PARENTS
 #define P2_COOP_MAX_PARENTS 16384
