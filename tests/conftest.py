@@ -17,6 +17,16 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a HIP GPU (MI355X); runs through libpil2_commit_hip.so")
 
 
+def pytest_collection_modifyitems(items):
+    """Tests that load the compiled reference come last. Where it is not built they fail,
+    and a run that stops at the first failure (-x) would end before all others."""
+    def loads_reference(item):
+        code = [item.function] + [d[-1].func for d in item._fixtureinfo.name2fixturedefs.values()]
+        return any("RefLib" in f.__code__.co_names for f in code if hasattr(f, "__code__"))
+
+    items.sort(key=loads_reference)
+
+
 @pytest.fixture(scope="session")
 def oracle():
     from oracle.oracle import Oracle

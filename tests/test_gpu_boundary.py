@@ -298,3 +298,21 @@ def test_wrapper_temporaries_on_a_side_stream(pc):
     _sync()
     for k in range(4):
         assert np.array_equal(pc.to_host(roots[k]), want[k]), k
+
+
+@pytest.mark.parametrize("nb,nbe,cols,arity", [(10, 12, 13, 3), (12, 13, 40, 4), (9, 10, 7, 2), (4, 5, 3, 3), (14, 17, 9, 2)])
+def test_commit_witness_matches_oracle(pc, oracle, nb, nbe, cols, arity):
+    """As test_commit_witness_matches_compiled_reference, where that is not built."""
+    n, ne = 1 << nb, 1 << nbe
+    trace = datagen.uniform(n * cols, 7050 + nb * 8 + arity).reshape(n, cols)
+    nt = oracle.tree_num_elements(ne, arity)
+    off_dst, off_mt = n * cols + 11, n * cols + 11 + ne * cols + 5
+    aux = np.full(off_mt + nt + 9, SENTINEL, dtype=np.uint64)
+    root = np.zeros(4, dtype=np.uint64)
+    pc.commit_witness(root, arity, nb, nbe, cols, trace, aux, off_dst, off_mt)
+    lde = oracle.lde(trace, ne)
+    tree = oracle.merkletree(lde, arity)
+    assert np.array_equal(aux[off_dst:off_dst + ne * cols], lde.reshape(-1))
+    assert np.array_equal(aux[off_mt:off_mt + nt], tree) and np.array_equal(root, tree[-4:])
+    assert (aux[:off_dst] == SENTINEL).all() and (aux[off_dst + ne * cols:off_mt] == SENTINEL).all()
+    assert (aux[off_mt + nt:] == SENTINEL).all()
