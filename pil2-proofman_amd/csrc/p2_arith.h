@@ -4,8 +4,9 @@
 // canonicalised once, when a digest leaves the kernel. Three forms are used:
 //   u64 word  any 64-bit value v (meaning v mod p);
 //   hz        halves form: two 64-bit accumulators (lo, hi) meaning lo + 2^32 hi,
-//             each below 2^41. The linear layers sum the 32-bit halves of words
-//             with small coefficients in it, with no carry chains at all;
+//             each below 2^48. The linear layers sum the 32-bit halves of words
+//             with small coefficients in it (below 2^41), with no carry chains at
+//             all, and the digit sums of the matrix cores come in it (gl_digits.h);
 //   lz        three 32-bit words (l0, l1, c) meaning l0 + 2^32 l1 + 2^64 c with a
 //             small carry count c (the partial rounds' round-constant addition).
 // Since 2^64 = 2^32 - 1 (mod p), both fold back to a word with one
@@ -29,8 +30,8 @@ struct lz {
 };
 
 // Halves form: two 64-bit accumulators (lo, hi) meaning lo + 2^32 hi, each below
-// 2^41. Linear combinations with small coefficients of the 32-bit halves of
-// 64-bit words stay far below 2^64, so they need no carry chains.
+// 2^48. Linear combinations with small coefficients of the 32-bit halves of
+// 64-bit words and sums of signed digits stay far below 2^64, so they need no carry chains.
 struct hz {
     uint64_t lo, hi;
 };
@@ -74,11 +75,11 @@ __device__ __forceinline__ uint64_t lz_fold(lz a)
     return gl_pack(r0, r1);
 }
 
-// Three halves-form values (lo, hi < 2^41) to congruent 64-bit words. With
+// Three halves-form values (lo, hi < 2^48) to congruent 64-bit words. With
 // hi = h0 + 2^32 h1 and 2^64 = 2^32 - 1 (mod p): r = lo + h1 (2^32 - 1) is
-// below 2^42 (one v_mad_u64_u32, no carry-out); then h0 is added to r's high
+// below 2^49 (one v_mad_u64_u32, no carry-out); then h0 is added to r's high
 // word, and a carry-out of that add (2^64) becomes + (2^32 - 1), which cannot
-// carry again since the wrapped value is below 2^42.
+// carry again since the wrapped value is below 2^49 (its high word below 2^17).
 __device__ __forceinline__ void hz_fold3(const hz *a, uint64_t *out)
 {
     uint64_t r[3], d[3];

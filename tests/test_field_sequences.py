@@ -79,3 +79,27 @@ def test_inverse_roots_are_negated_powers_of_two():
     assert pow(w16, 16, P) == 1 and pow(w16, 8, P) == P - 1
     for k in range(1, 8):
         assert pow(w16, 16 - k, P) == (P - pow(2, 96 - 12 * k, P)) % P
+
+
+def _halves_fold(lo, hi):
+    """hz_fold, word by word: (lo, hi) meaning lo + 2^32 hi to a congruent 64-bit word."""
+    r = lo + (hi >> 32) * M32
+    assert r < 1 << 64  # the multiply-add's carry is dropped
+    r0, r1 = r & M32, r >> 32
+    r1 += hi & M32
+    c, r1 = r1 >> 32, r1 & M32
+    r0 -= c
+    b, r0 = int(r0 < 0), r0 & M32
+    r1 += c & (b ^ 1)
+    assert r1 >> 32 == 0  # and so is this one
+    return r1 << 32 | r0
+
+
+def test_halves_fold_up_to_the_digit_sums():
+    """Accumulators of the linear layers (below 2^41) and of digit sums (below 2^48)."""
+    rng = random.Random(11)
+    edge = [0, 1, M32 - 1, M32, M32 + 1, 1 << 41, (1 << 48) - 1, (1 << 48) - (1 << 32), (1 << 48) - (1 << 32) + 1,
+            ((1 << 16) - 1 << 32) | M32 - 1]
+    pairs = [(a, b) for a in edge for b in edge] + [(rng.randrange(1 << 48), rng.randrange(1 << 48)) for _ in range(20000)]
+    for lo, hi in pairs:
+        assert (_halves_fold(lo, hi) - lo - (hi << 32)) % P == 0, (lo, hi)
