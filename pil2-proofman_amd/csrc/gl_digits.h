@@ -74,18 +74,20 @@ __device__ __forceinline__ void gl_mac16(gl_v4i &acc, const gl_v4i &a, const gl_
 // that is free to the assembly's outputs at once. Assembly near matrix instructions thus
 // writes only registers that an instruction of the compiler's has written before: its
 // vector outputs start as operands ("+v"), and a value that starts anew is a product in C.
-// tests/test_isa_hazards.py looks for early accesses in the built code. (Time: the same,
-// LDE and commits within 1 %.)
+// tests/test_isa_hazards.py looks for early accesses in the built code. (Time against outputs of the assembly's own: LDE of
+// 2^22 x 128 to 2^24 30.8 -> 30.6 ms, 2^19 x 64 to 2^20 1,015 -> 1,026 us, commits the same.)
 
 // e 2^16 + k (the factor is hidden from the compiler: shifts and adds take two more), k
-// a lane's own or (SK) in scalar registers
+// a lane's own or (SK) in scalar registers. An instruction takes one scalar operand: with
+// the factor in the other kind of register k stays where it is (a scalar factor for both
+// kinds: constants k held in vector registers, 60 of 128 spilled in block passes).
 template <bool SK> __device__ __forceinline__ uint64_t gl_mad_64k(int e, uint64_t k)
 {
     int c16 = 65536;
     if constexpr (SK)
-        asm("" : "+v"(c16), "+s"(k));
+        asm("" : "+v"(c16));
     else
-        asm("" : "+s"(c16));
+        asm volatile("" : "+s"(c16));
     return (uint64_t)((int64_t)e * c16) + k;
 }
 // e + k

@@ -19,7 +19,9 @@
 // are 20 percent busy; waiting (LDS, twiddles, barriers) is what is left, so registers are
 // held to 128 for four waves a SIMD: with 256 and two waves the same rounds took 16.8,
 // 14.3 and 4.1 ms. Each value spilled at 128 is 256 bytes of memory traffic a wave; the
-// fences below keep the pieces of an unrolled round apart for that reason.
+// fences below keep the pieces of an unrolled round apart for that reason. What still
+// spills: 6 to 12 registers a line in the block pass of blowup 4, 4 to 8 of blowup 8, and in
+// the strided inverse of 2^8 points 8, of the matrix.
 #pragma once
 #include "gl_digits.h"
 

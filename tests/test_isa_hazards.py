@@ -41,8 +41,10 @@ def _instruction(op, operands, address, target):
         writes = reads = writes | reads
     elif op.startswith(("v_fmac", "v_writelane")):
         reads = reads | writes
-    if not op.startswith("v_"):
-        writes = reads = set()
+    if not op.startswith("v_"):  # of the others only the results of scalar instructions count
+        reads = set()
+        if not op.startswith("s_") or op.startswith(("s_cmp", "s_bitcmp", "s_cbranch", "s_waitcnt", "s_nop")):
+            writes = set()
     return Instruction(op, operands, writes, reads, address, target)
 
 
@@ -82,6 +84,8 @@ def early(code, at, start, rules):
                 for (name, _, wait, w, r), s in zip(rules, sets):
                     if waited < wait and s & ((i.writes if w else set()) | (i.reads if r else set())):
                         found.append("%s after %d: %s %s" % (name, waited, i.op, ", ".join(i.operands)))
+                sets = tuple(s - i.writes for s in sets)
+            else:
                 sets = tuple(s - i.writes for s in sets)
             waited += int(i.operands[0], 0) + 1 if i.op == "s_nop" else 1
             if i.op in ("s_endpgm", "s_setpc_b64", "s_swappc_b64"):
@@ -160,7 +164,7 @@ MASK_WAIT = 2
 def mask_hazards(code):
     out, at = [], {i.address: k for k, i in enumerate(code)}
     for k, i in enumerate(code):
-        masks = {r for r in i.writes if r[0] == "s"}
+        masks = {r for r in i.writes if r[0] == "s"} if i.op.startswith("v_") else set()
         if masks:
             out += early(code, at, k, [("mask", masks, MASK_WAIT, False, True)])
     return out
