@@ -245,8 +245,8 @@ int64_t pil2hip_commit_batch(const Pil2CommitJob *jobs, uint64_t n_jobs, uint32_
  *                     (radix 4, 8, 16); the strided passes always take the fewest
  *                     rounds of at most 4 bits
  *                     (tile and radix concern shapes whose rounds stay on the VALU:
- *                     blowups above 8, lines below 2^8 or transforms above 2^24 rows;
- *                     the others have one plan)
+ *                     blowups above 8, fewer than 2^8 rows, fewer than 2^10 or more
+ *                     than 2^24 extended rows; the others have one plan)
  *   coop_max_parents  tree levels with at most this many parents hash with 16 lanes
  *                     per permutation, larger levels with one lane per parent
  * The plain entry points and fields left 0 use {-, 13, 4, 16384}. */

@@ -196,8 +196,9 @@ static int64_t check_arity(uint64_t arity)
     return 0;
 }
 
-// Tile and radix matter only to the shapes whose transform rounds stay on the VALU
-// (blowups above 8, above 2^24 rows): 2^13 tiles, two blocks per CU, and radix-16 rounds
+// Tile and radix matter only to the shapes whose transform rounds stay on the VALU (blowups
+// above 8, below 2^8 rows, below 2^10 or above 2^24 extended rows): 2^13 tiles, two blocks per
+// CU, and radix-16 rounds
 static const Pil2CommitPlan kDefaultPlan = {1, 13, 4, P2_COOP_MAX_PARENTS};
 
 static int64_t lde_impl(uint64_t *d_lde, const uint64_t *d_trace, uint64_t *d_scratch, uint64_t nBits,
