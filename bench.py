@@ -53,6 +53,8 @@ CLOCK_HZ = 2.4e9
 # Poseidon2 field multiplications per permutation (algorithmic count):
 # 8 full rounds x W x 4 (x^7) + 22 partial rounds x (4 + W)
 MULS_PER_PERM = {8: 8 * 8 * 4 + 22 * 12, 12: 8 * 12 * 4 + 22 * 16, 16: 8 * 16 * 4 + 22 * 20}
+# those of them on the VALU: the S-boxes (the partial rounds' diagonals are on the matrix cores)
+VALU_MULS_PER_PERM = {w: (8 * w + 22) * 4 for w in (8, 12, 16)}
 
 
 def host_info():
@@ -211,7 +213,8 @@ def _leaf_roofline(width, perms, leaf_ms, leaf_bytes, traffic, launches):
     """VALU roofline of the Poseidon2 leaf kernel: algorithmic Goldilocks
     multiplications (736 per W12 permutation) against the rate at which the VALU
     can issue the four 32x32->64 partial products each one needs (v_mad_u64_u32
-    at the single-issue lane rate), i.e. a products-only ceiling."""
+    at the single-issue lane rate), i.e. a products-only ceiling. The share of the
+    measured product rate counts the products that the VALU executes."""
     leaf_s = leaf_ms / 1e3
     muls_per_s = perms * MULS_PER_PERM[width] / leaf_s
     mul_peak = VALU_PEAK_TOPS / 4.0  # T mul/s
@@ -224,9 +227,11 @@ def _leaf_roofline(width, perms, leaf_ms, leaf_bytes, traffic, launches):
                                                                              VALU_PEAK_TOPS),
         "perm_per_s": perms / leaf_s,
         "mul_peak_measured": round(measured_mul_peak()[0], 4),
-        "frac_of_measured_mul_peak": round(muls_per_s / 1e12 / measured_mul_peak()[0], 4),
+        "valu_muls_per_perm": VALU_MULS_PER_PERM[width],
+        "frac_of_measured_mul_peak": round(perms * VALU_MULS_PER_PERM[width] / leaf_s / 1e12 / measured_mul_peak()[0], 4),
         "mul_peak_note": "pil2hip_mul_peak: the kernel's own reduced product (11 single-rate instructions), "
-                         "18 independent chains per lane, 2^21 lanes",
+                         "18 independent chains per lane, 2^21 lanes; its share counts the valu_muls_per_perm "
+                         "products on the VALU, the other ones run on the matrix cores",
         "hbm_achieved_GBs": leaf_bytes / leaf_s / 1e9, "hbm_frac": leaf_bytes / leaf_s / 1e9 / HBM_PEAK_GBS,
         "traffic": traffic,
         "avg_ms": leaf_ms / launches,
@@ -258,7 +263,8 @@ def _lde_valu_roofline(nb, nbe, cols, lde_ms, config):
            "frac": round(achieved / peak, 4), "butterflies": bfly,
            "floor_ms": round(bfly * INSTR_PER_BUTTERFLY / (VALU_PEAK_TOPS * 1e12) * 1e3, 3),
            "model": "radix-2 butterflies of the iNTT (N/2 log N) and the forward NTT after zero extension "
-                    "(NExt/2 log N), %d single-rate instructions each at %.1f T lane-op/s"
+                    "(NExt/2 log N), %d single-rate instructions each at %.1f T lane-op/s if all were on the "
+                    "VALU (rounds of four index bits are on the matrix cores)"
                     % (INSTR_PER_BUTTERFLY, VALU_PEAK_TOPS)}
     cyc, lanes = 0.0, 0.0
     for k in _lde_kernels(nb, nbe, cols):
@@ -1106,7 +1112,8 @@ def run_plain(args, cfg):
         "per_pass_achieved": pass_bytes / (lde_ms / 1e3) / 1e9,
         "per_pass_frac": pass_bytes / (lde_ms / 1e3) / 1e9 / HBM_PEAK_GBS,
         "traffic": lde_traffic, "avg_ms": lde_ms,
-        "limited_by": "valu: the field arithmetic's instruction count, not HBM (the 'valu' object)",
+        "limited_by": "waiting: LDS, twiddle reads and barriers between rounds on the matrix cores, at one or two "
+                      "blocks per CU; neither VALU issue (the 'valu' object) nor HBM is full",
         "valu": _lde_valu_roofline(nb, nbe, cols, lde_ms, args.config),
     }
     out = {
